@@ -24,9 +24,14 @@ OBJDIR = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libspacecharge_mi355.so")
 ARCH = "gfx950"
 
-SOURCES = ["sc_api.cpp", "sc_particles.hip", "sc_deposit.hip", "sc_green.hip", "sc_solve.hip",
-           "sc_solve_fast.hip"]
-HEADERS = ["sc_internal.h", "sc_fft_dev.h", "sc_fft_reg.h", "sc_solve_common.h"]
+# (source, object suffix, extra flags); the transform kernels, one set per
+# length and mesh type, compile in parts that build in parallel
+UNITS = [("sc_solve_mix.hip", f"_{k}", [f"-DSC_MIX_PART={k}"]) for k in range(4)]
+UNITS += [("sc_green.hip", f"_{k}", [f"-DSC_GREEN_PART={k}"]) for k in range(2)]
+UNITS += [("sc_api.cpp", "", []), ("sc_particles.hip", "", []), ("sc_deposit.hip", "", []),
+          ("sc_solve.hip", "", []), ("sc_solve_fast.hip", "", [])]
+HEADERS = ["sc_internal.h", "sc_fft_dev.h", "sc_fft_reg.h", "sc_fft_mix.h",
+           "sc_solve_common.h"]
 
 
 def hipcc() -> str:
@@ -49,9 +54,10 @@ COMMON = [
 ]
 
 
-def _compile(src: str) -> str:
-    obj = os.path.join(OBJDIR, os.path.splitext(src)[0] + ".o")
-    cmd = [hipcc()] + COMMON + ["-c", os.path.join(CSRC, src), "-o", obj]
+def _compile(unit) -> str:
+    src, suffix, flags = unit
+    obj = os.path.join(OBJDIR, os.path.splitext(src)[0] + suffix + ".o")
+    cmd = [hipcc()] + COMMON + flags + ["-c", os.path.join(CSRC, src), "-o", obj]
     if src.endswith(".cpp"):
         cmd[1:1] = ["-x", "hip"]
     r = subprocess.run(cmd, capture_output=True, text=True)
@@ -63,8 +69,8 @@ def _compile(src: str) -> str:
 def build(verbose: bool = False) -> str:
     """Compile every source (always) and link the shared library; returns its path."""
     os.makedirs(OBJDIR, exist_ok=True)
-    with cf.ThreadPoolExecutor(max_workers=min(len(SOURCES), os.cpu_count() or 1)) as ex:
-        objs = list(ex.map(_compile, SOURCES))
+    with cf.ThreadPoolExecutor(max_workers=min(len(UNITS), os.cpu_count() or 1)) as ex:
+        objs = list(ex.map(_compile, UNITS))
     tmp = LIB + ".tmp"
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp] + objs
     r = subprocess.run(cmd, capture_output=True, text=True)

@@ -1069,6 +1069,7 @@ int launch_deposit_binned_multi(Mesh *m, int pdt, const void *x, const void *y, 
         g.dl[a] = lo ? dl[a] : 1.0;
     }
     if (int rc = ensure_bins(m, n, pdt, g.tx * g.ty * g.tz, nchan)) return rc;
+    note_particles(m, pdt);
     if (nchan > 1) {
         DepositBins &B = m->bins;
         const size_t need = (size_t)2 * n * pdt;
@@ -1320,6 +1321,7 @@ int launch_deposit_grouped(Ctx *ctx, Mesh *const *ms, int nb, int pdt, const voi
     if (int rc = ensure_group_table(ctx, group_table_bytes())) return rc;
     for (int b = 0; b < nb; ++b)
         if (int rc = ensure_bins(ms[b], n[b], pdt, geos[b].tx * geos[b].ty * geos[b].tz, 1)) return rc;
+    for (int b = 0; b < nb; ++b) note_particles(ms[b], pdt);
     // where each mesh's deposit starts on the stream (a later solve's Green
     // build on the side stream waits for it, as after launch_deposit)
     for (int b = 0; b < nb; ++b)

@@ -34,7 +34,6 @@
 #include <cstring>
 #include <type_traits>
 
-#include "sc_fft_reg.h"
 #include "sc_solve_common.h"
 
 namespace sc {
@@ -826,6 +825,253 @@ k_green_3r(const T *__restrict__ R, T *__restrict__ Gf, cpx<T> *__restrict__ Gi,
     }
 }
 
+// ---- the same passes on the mixed-radix lengths of sc_fft_mix.h ----
+using mix::Shape;
+
+template <typename T, int L>
+__global__ void __launch_bounds__((Shape<T, L>::THREADS))
+k_green_1m(const double *__restrict__ F, T *__restrict__ R, const cpx<T> *__restrict__ twg,
+           GreenArgs a, const SBunch *__restrict__ tab, int per)
+{
+    using S = Shape<T, L>;
+    constexpr int E = S::E, TPP = S::TPP, NB = S::NB;
+    __shared__ cpx<T> tw[L];
+    __shared__ cpx<T> lds[NB * reg::padded<L, E>()];
+    // one bunch: workgroups in XCD order over the whole grid (pencils of
+    // plane k + 1 read the F rows of plane k's pencils a few workgroups
+    // earlier, which then sit on the same XCD and its L2)
+    const SBunch *sb = nullptr;
+    int bx, q;
+    if (tab) {
+        bx = group_block(tab, per, sb);
+        q = (int)blockIdx.y;
+    } else {
+        const int task = xcd_task((int)(blockIdx.x + blockIdx.y * gridDim.x),
+                                  (int)(gridDim.x * gridDim.y));
+        bx = task % (int)gridDim.x;
+        q = task / (int)gridDim.x;
+    }
+    if (sb) {
+        F = sb->F;
+        R = static_cast<T *>(sb->R);
+    }
+    for (int i = threadIdx.x; i < L; i += S::THREADS) tw[i] = gld(twg + i);
+    const int c = comp_of(a, q), image = q / 3;
+    const int nx = a.d.nx, ny = a.d.ny, Kx = a.d.Kx, Kp = a.d.Kp;
+    const int bpairs = (ny + 1) / 2;
+    const int npencils = z_cells(a, image) * bpairs;
+    const int b = threadIdx.x / TPP, j = threadIdx.x % TPP;
+    const int P = bx * NB + b;
+    const bool live = P < npencils;
+    const int k = live ? P / bpairs : 0, ya = live ? 2 * (P - k * bpairs) : 0;
+    const bool hasb = ya + 1 < ny;
+    const gbl<double> *Fq = (const gbl<double> *)(F + f_off(a, q));
+    const T sgn = (c == 0) ? (T)-1 : (T)1;
+    // The extension's upper half (e > nx) mirrors cells nx - 1 .. 1, so each
+    // cell row is differenced once (e < nx, the first E/2 registers when
+    // L = 2 nx) and the mirror is read back through this pencil's LDS slice.
+    cpx<T> *row = lds + b * reg::padded<L, E>();
+    cpx<T> v[E];
+    // F rows ya, ya+1, ya+2 (clamped: without a second row the third is
+    // unused) of planes k, k+1, loaded without branches two cells at a time
+    // (one when E / 2 is odd) so that their 24 loads are in flight together
+    const int64_t sy = nx + 1, sz = (int64_t)(nx + 1) * (ny + 1);
+    const int yr[3] = {ya, ya + 1, ya + 2 <= ny ? ya + 2 : ny};
+    constexpr int kCells = (E / 2) % 2 == 0 ? 2 : 1;
+#pragma unroll
+    for (int r0 = 0; r0 < E / 2; r0 += kCells) {
+        double f[kCells][3][2][2];  // [cell][y][z][x]
+#pragma unroll
+        for (int u = 0; u < kCells; ++u) {
+            const int e = j + (r0 + u) * TPP;
+#pragma unroll
+            for (int yy = 0; yy < 3; ++yy)
+#pragma unroll
+                for (int zz = 0; zz < 2; ++zz) {
+                    const gbl<double> *p = Fq + e + sy * yr[yy] + sz * (k + zz);
+                    f[u][yy][zz][0] = p[0];
+                    f[u][yy][zz][1] = p[1];
+                }
+        }
+#pragma unroll
+        for (int u = 0; u < kCells; ++u) {
+            const int r = r0 + u;
+            const double ga = diff8v(f[u][0][0][0], f[u][0][0][1], f[u][0][1][0], f[u][0][1][1],
+                                     f[u][1][0][0], f[u][1][0][1], f[u][1][1][0], f[u][1][1][1]);
+            const double gb = diff8v(f[u][1][0][0], f[u][1][0][1], f[u][1][1][0], f[u][1][1][1],
+                                     f[u][2][0][0], f[u][2][0][1], f[u][2][1][0], f[u][2][1][1]);
+            v[r].x = live ? (T)ga : (T)0;
+            v[r].y = (live && hasb) ? (T)gb : (T)0;
+            row[j + r * TPP] = v[r];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = E / 2; r < E; ++r) {
+        const int e = j + r * TPP;
+        const cpx<T> m = row[L - e];  // e >= nx; e == nx reads row[nx], unused
+        v[r] = e == nx ? cpx<T>{(T)0, (T)0} : cpx<T>{sgn * m.x, sgn * m.y};
+    }
+    mix::fft<T, L, E, -1>(v, j, row, 1, tw);
+    if (live) {
+        gbl<T> *Rq = (gbl<T> *)(R + r_off(a, q));
+#pragma unroll
+        for (int r = 0; r <= E / 2; ++r) {
+            const int kx = j + r * TPP;
+            if (r < E / 2 || kx == nx) {
+                T ra, rb;
+                unpack_pair(v[r], c == 0, ra, rb);
+                Rq[((size_t)k * (ny + 1) + ya) * Kp + kx] = ra;
+                if (hasb) Rq[((size_t)k * (ny + 1) + ya + 1) * Kp + kx] = rb;
+            }
+        }
+    }
+}
+
+template <typename T, int L>
+__global__ void __launch_bounds__((Shape<T, L>::THREADS))
+k_green_2m(T *__restrict__ R, const cpx<T> *__restrict__ twg, GreenArgs a,
+           const SBunch *__restrict__ tab, int per)
+{
+    using S = Shape<T, L>;
+    constexpr int E = S::E, TPP = S::TPP, NB = S::NB;
+    __shared__ cpx<T> tw[L];
+    __shared__ cpx<T> lds[NB * L];
+    const SBunch *sb;
+    const int bx = group_block(tab, per, sb);
+    if (sb) R = static_cast<T *>(sb->R);
+    const int q = blockIdx.z, c = comp_of(a, q), image = q / 3;
+    const int k = blockIdx.y;
+    if (k >= z_cells(a, image)) return;  // uniform over the workgroup
+    for (int i = threadIdx.x; i < L; i += S::THREADS) tw[i] = gld(twg + i);
+    const int ny = a.d.ny, Kx = a.d.Kx, Kp = a.d.Kp;
+    const int b = threadIdx.x % NB, j = threadIdx.x / NB;
+    const int kxa = 2 * (bx * NB + b), kxb = kxa + 1;
+    gbl<T> *Rrow = (gbl<T> *)(R + r_off(a, q) + (size_t)k * (ny + 1) * Kp);
+    const T sgn = (c == 1) ? (T)-1 : (T)1;
+    // every load is in range (clamped row and column) and issued without a
+    // branch, so a lane's loads are all in flight together; the selects
+    // below apply the extension and the bounds
+    const int kxa_c = kxa < Kx ? kxa : Kx - 1, kxb_c = kxb < Kx ? kxb : Kx - 1;
+    T ra[E], rb[E];
+#pragma unroll
+    for (int r = 0; r < E; ++r) {
+        const int e = j + r * TPP;
+        const int y = e < ny ? e : (e == ny ? 0 : L - e);
+        ra[r] = Rrow[(size_t)y * Kp + kxa_c];
+        rb[r] = Rrow[(size_t)y * Kp + kxb_c];
+    }
+    cpx<T> v[E];
+#pragma unroll
+    for (int r = 0; r < E; ++r) {
+        const int e = j + r * TPP;
+        const T s = e < ny ? (T)1 : sgn;
+        v[r].x = (kxa < Kx && e != ny) ? s * ra[r] : (T)0;
+        v[r].y = (kxb < Kx && e != ny) ? s * rb[r] : (T)0;
+    }
+    mix::fft<T, L, E, -1>(v, j, lds + b, NB, tw);
+#pragma unroll
+    for (int r = 0; r <= E / 2; ++r) {
+        const int ky = j + r * TPP;
+        if (r < E / 2 || ky == ny) {
+            T ra, rb;
+            unpack_pair(v[r], c == 1, ra, rb);
+            if (kxa < Kx) Rrow[(size_t)ky * Kp + kxa] = ra;
+            if (kxb < Kx) Rrow[(size_t)ky * Kp + kxb] = rb;
+        }
+    }
+}
+
+template <typename T, int L>
+__global__ void __launch_bounds__((Shape<T, L>::THREADS))
+k_green_3m(const T *__restrict__ R, T *__restrict__ Gf, cpx<T> *__restrict__ Gi,
+           const cpx<T> *__restrict__ twg, GreenArgs a, const SBunch *__restrict__ tab, int per)
+{
+    using S = Shape<T, L>;
+    constexpr int E = S::E, TPP = S::TPP, NB = S::NB;
+    __shared__ cpx<T> tw[L];
+    __shared__ cpx<T> lds[NB * L];
+    const SBunch *sb;
+    const int bx = group_block(tab, per, sb);
+    if (sb) {
+        R = static_cast<const T *>(sb->R);
+        Gf = static_cast<T *>(sb->Gf);
+        Gi = static_cast<cpx<T> *>(sb->Gi);
+        green_from_table(a, sb);
+    }
+    for (int i = threadIdx.x; i < L; i += S::THREADS) tw[i] = gld(twg + i);
+    const int q = blockIdx.z, c = comp_of(a, q), image = q / 3;
+    const int ky = blockIdx.y;
+    const int nz = a.d.nz, Kx = a.d.Kx, Kp = a.d.Kp, ny1 = a.d.ny + 1;
+    const int b = threadIdx.x % NB, j = threadIdx.x / NB;
+    const int kxa = 2 * (bx * NB + b), kxb = kxa + 1;
+    const gbl<T> *Rq = (const gbl<T> *)(R + r_off(a, q));
+    const T sgn = (c == 2) ? (T)-1 : (T)1;
+    // loads clamped in range and issued without branches (see k_green_2m)
+    const int kxa_c = kxa < Kx ? kxa : Kx - 1, kxb_c = kxb < Kx ? kxb : Kx - 1;
+    T ra[E], rb[E], sc[E];
+    bool on[E];
+#pragma unroll
+    for (int r = 0; r < E; ++r) {
+        const int e = j + r * TPP;
+        int cell = 0;
+        T s = (T)1;
+        on[r] = e != nz;  // slot e == nz is zero
+        if (!image) {
+            if (e != nz) {
+                cell = e < nz ? e : L - e;
+                s = e < nz ? (T)1 : sgn;
+            }
+        } else if (e != nz) {
+            // slot e holds displacement e (e < nz) or e - L (e > nz); row = displacement + nz - 1
+            cell = e < nz ? e + nz - 1 : e - nz - 1;
+        }
+        const gbl<T> *row = Rq + ((size_t)cell * ny1 + ky) * Kp;
+        ra[r] = row[kxa_c];
+        rb[r] = row[kxb_c];
+        sc[r] = s;
+    }
+    cpx<T> v[E];
+#pragma unroll
+    for (int r = 0; r < E; ++r) {
+        v[r].x = (kxa < Kx && on[r]) ? sc[r] * ra[r] : (T)0;
+        v[r].y = (kxb < Kx && on[r]) ? sc[r] * rb[r] : (T)0;
+    }
+    mix::fft<T, L, E, -1>(v, j, lds + b, NB, tw);
+    const T scale = (T)green_scale(a, c);
+    if (!image) {
+        gbl<T> *G = (gbl<T> *)(Gf + (size_t)(q % 3) * (nz + 1) * ny1 * Kp);
+#pragma unroll
+        for (int r = 0; r <= E / 2; ++r) {
+            const int kz = j + r * TPP;
+            if (r < E / 2 || kz == nz) {
+                T ra, rb;
+                unpack_pair(v[r], c == 2, ra, rb);
+                gbl<T> *row = G + ((size_t)kz * ny1 + ky) * Kp;
+                if (kxa < Kx) row[kxa] = ra * scale;
+                if (kxb < Kx) row[kxb] = rb * scale;
+            }
+        }
+    } else {
+        // the separation needs X[-kz], held by another lane: go through LDS
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < E; ++r) lds[b + (j + r * TPP) * NB] = v[r];
+        __syncthreads();
+        cpx<T> *G = Gi + (size_t)(q % 3) * L * ny1 * Kp;
+        const T h = (T)0.5 * scale;
+#pragma unroll
+        for (int r = 0; r < E; ++r) {
+            const int kz = j + r * TPP;
+            const cpx<T> X = v[r];
+            const cpx<T> Y = lds[b + (kz == 0 ? 0 : L - kz) * NB];
+            cpx<T> *row = G + ((size_t)kz * ny1 + ky) * Kp;
+            if (kxa < Kx) gst(row + kxa, cpx<T>{(X.x + Y.x) * h, (X.y - Y.y) * h});
+            if (kxb < Kx) gst(row + kxb, cpx<T>{(X.y + Y.y) * h, (Y.x - X.x) * h});
+        }
+    }
+}
+
 template <typename T, int L>
 void green_pass_r(int pass, dim3 grid, hipStream_t st, const Workspace &ws, const GreenArgs &a,
                   const cpx<T> *tw)
@@ -839,6 +1085,23 @@ void green_pass_r(int pass, dim3 grid, hipStream_t st, const Workspace &ws, cons
                            (const SBunch *)nullptr, 0);
     else
         hipLaunchKernelGGL((k_green_3r<T, L>), grid, dim3(kRThreads), 0, st, (const T *)R,
+                           static_cast<T *>(ws.Gf), static_cast<cpx<T> *>(ws.Gi), tw, a,
+                           (const SBunch *)nullptr, 0);
+}
+
+template <typename T, int L>
+void green_pass_m(int pass, dim3 grid, hipStream_t st, const Workspace &ws, const GreenArgs &a,
+                  const cpx<T> *tw)
+{
+    T *R = static_cast<T *>(ws.R);
+    const dim3 block(Shape<T, L>::THREADS);
+    if (pass == 1)
+        hipLaunchKernelGGL((k_green_1m<T, L>), grid, block, 0, st, (const double *)ws.F, R, tw, a,
+                           (const SBunch *)nullptr, 0);
+    else if (pass == 2)
+        hipLaunchKernelGGL((k_green_2m<T, L>), grid, block, 0, st, R, tw, a, (const SBunch *)nullptr, 0);
+    else
+        hipLaunchKernelGGL((k_green_3m<T, L>), grid, block, 0, st, (const T *)R,
                            static_cast<T *>(ws.Gf), static_cast<cpx<T> *>(ws.Gi), tw, a,
                            (const SBunch *)nullptr, 0);
 }
@@ -866,6 +1129,13 @@ bool green_pass_fast(int pass, int L, int ncomp, const Dims &d, int cath, hipStr
         SC_GREEN_CASE(256)
         SC_GREEN_CASE(512)
 #undef SC_GREEN_CASE
+#define X(LL)                                                                  \
+    case LL:                                                                   \
+        green_pass_m<T, LL>(pass, grid_for(Shape<T, LL>::NB), st, ws, a, tw);  \
+        return true;
+        SC_MIX_SHORT(X)
+        SC_MIX_LONG(X)
+#undef X
     default: return false;
     }
 }
@@ -920,9 +1190,9 @@ int build_green(Mesh *m, const double dl[3], double gamma, double offz, int mode
                                ws.F, a, (const SBunch *)nullptr, 0);
         launch_end(ctx, K_GREEN_F);
     }
-    const bool fast_ok = !m->generic_transforms;
     launch_begin(ctx, K_GREEN_X);
-    if (!(fast_ok && green_pass_fast<T>(1, d.Lx, ncomp, d, cath, st, ws, a, twx))) {
+    if (engine_of(m, d.Lx, false) == kGeneric ||
+        !green_pass_fast<T>(1, d.Lx, ncomp, d, cath, st, ws, a, twx)) {
         with_fft_elems<T>(d.Lx, [&](auto e, auto t) {
             constexpr int E = decltype(e)::value, NT = decltype(t)::value;
             const int nb = pick_nb(d.Lx, E * NT, 16);
@@ -936,7 +1206,8 @@ int build_green(Mesh *m, const double dl[3], double gamma, double offz, int mode
     launch_end(ctx, K_GREEN_X);
     const int kp = (d.Kx + 1) / 2;
     launch_begin(ctx, K_GREEN_Y);
-    if (!(fast_ok && green_pass_fast<T>(2, d.Ly, ncomp, d, cath, st, ws, a, twy))) {
+    if (engine_of(m, d.Ly, false) == kGeneric ||
+        !green_pass_fast<T>(2, d.Ly, ncomp, d, cath, st, ws, a, twy)) {
         with_fft_elems<T>(d.Ly, [&](auto e, auto t) {
             constexpr int E = decltype(e)::value, NT = decltype(t)::value;
             const int nb = pick_nb(d.Ly, E * NT, 16);
@@ -948,7 +1219,8 @@ int build_green(Mesh *m, const double dl[3], double gamma, double offz, int mode
     }
     launch_end(ctx, K_GREEN_Y);
     launch_begin(ctx, K_GREEN_Z);
-    if (!(fast_ok && green_pass_fast<T>(3, d.Lz, ncomp, d, cath, st, ws, a, twz))) {
+    if (engine_of(m, d.Lz, false) == kGeneric ||
+        !green_pass_fast<T>(3, d.Lz, ncomp, d, cath, st, ws, a, twz)) {
         with_fft_elems<T>(d.Lz, [&](auto e, auto t) {
             constexpr int E = decltype(e)::value, NT = decltype(t)::value;
             const int nb = pick_nb(d.Lz, E * NT, 16);
@@ -1015,22 +1287,48 @@ void build_green_grouped(const Mesh *m0, int nb, const SBunch *tab, double gamma
                                    (cpx<T> *)nullptr, tw[2], a, tab, per);
             }
         };
+        auto gom = [&](auto lc) {
+            constexpr int LL = decltype(lc)::value;
+            constexpr int NB = Shape<T, LL>::NB;
+            if (pass == 1) {
+                const int per = div_up(zc * ((d.ny + 1) / 2), NB);
+                hipLaunchKernelGGL((k_green_1m<T, LL>), dim3(per * nb, ncomp), dim3(Shape<T, LL>::THREADS), 0, st,
+                                   (const double *)nullptr, (T *)nullptr, tw[0], a, tab, per);
+            } else if (pass == 2) {
+                const int per = div_up(kp, NB);
+                hipLaunchKernelGGL((k_green_2m<T, LL>), dim3(per * nb, zc, ncomp), dim3(Shape<T, LL>::THREADS), 0,
+                                   st, (T *)nullptr, tw[1], a, tab, per);
+            } else {
+                const int per = div_up(kp, NB);
+                hipLaunchKernelGGL((k_green_3m<T, LL>), dim3(per * nb, d.ny + 1, ncomp),
+                                   dim3(Shape<T, LL>::THREADS), 0, st, (const T *)nullptr, (T *)nullptr,
+                                   (cpx<T> *)nullptr, tw[2], a, tab, per);
+            }
+        };
         switch (L) {
         case 32: go(std::integral_constant<int, 32>{}); break;
         case 64: go(std::integral_constant<int, 64>{}); break;
         case 128: go(std::integral_constant<int, 128>{}); break;
         case 256: go(std::integral_constant<int, 256>{}); break;
         case 512: go(std::integral_constant<int, 512>{}); break;
+#define X(LL) \
+        case LL: gom(std::integral_constant<int, LL>{}); break;
+        SC_MIX_SHORT(X)
+        SC_MIX_LONG(X)
+#undef X
         default: break;  // the caller groups only supported lengths
         }
     }
 }
 
+// one mesh type per compilation (SC_GREEN_PART, see build.py)
+#if SC_GREEN_PART == 0
 template void build_green_grouped<float>(const Mesh *, int, const SBunch *, double, int, hipStream_t);
+template int build_green<float>(Mesh *, const double[3], double, double, int);
+#else
 template void build_green_grouped<double>(const Mesh *, int, const SBunch *, double, int,
                                           hipStream_t);
-
-template int build_green<float>(Mesh *, const double[3], double, double, int);
 template int build_green<double>(Mesh *, const double[3], double, double, int);
+#endif
 
 }  // namespace sc

@@ -157,6 +157,7 @@ struct Ctx {
 // Device workspace of one mesh (lazy, like src/mesh.jl:49-72).
 struct Workspace {
     bool ready = false;
+    bool smooth = false;  // transform lengths: see smooth_lengths (fixed when the workspace is made)
     int dtype = 0;
     int64_t bytes = 0;
     // spectra in the mesh type T: A = rho after the x and y transforms,
@@ -227,6 +228,7 @@ struct Mesh {
     bool owns = false;
     bool green_reuse = false;
     bool generic_transforms = false;  // diagnostic: skip the register-resident engine
+    bool f64_particles = false;       // a Float32 mesh that Float64 particles were deposited on
     Workspace ws;
     DepositBins bins;
     void *efi = nullptr;  // node-interleaved field for the interpolation gather
@@ -244,6 +246,13 @@ struct Mesh {
     int chunk_log2 = 13;
     int slice_log2 = 12;
 };
+
+// Remembers the widest particles deposited on a Float32 mesh (the lengths of
+// its transforms, smooth_lengths).
+inline void note_particles(Mesh *m, int pdt)
+{
+    if (pdt == SC_F64 && m->dtype == SC_F32) m->f64_particles = true;
+}
 
 constexpr int kChunkLog2Min = 10, kChunkLog2Max = 14;
 constexpr int kSliceLog2Min = 10, kSliceLog2Max = 13;

@@ -642,6 +642,7 @@ int launch_deposit_to(Mesh *m, int pdt, const void *x, const void *y, const void
     const int rc = launch_deposit_binned(m, pdt, x, y, z, q, n, lo, dl, clear, out);
     if (rc != SC_ERR_UNSUPPORTED) return rc;
     // more tiles than the binned path holds: one atomic per node contribution
+    note_particles(m, pdt);
     if (clear) {
         if (int rc2 = launch_clear(m->ctx, out, rho_bytes)) return rc2;
     }

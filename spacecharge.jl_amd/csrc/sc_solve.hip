@@ -424,10 +424,14 @@ int run_solve(Mesh *m, const double lo[3], const double hi[3], const double dl[3
         std::memcpy(ws.g_key, key, sizeof(key));
     }
 
-    // Each transform kernel runs on the register-resident engine when its
-    // length is a supported power of two, else on the generic LDS engine.
-    const bool fast_ok = !m->generic_transforms && !dims_padded(d);
-    auto fast = [&](int which) { return fast_ok && launch_fast<T>(m, which, io); };
+    // Each transform kernel runs on a register-resident engine when one
+    // supports its length, else on the generic LDS engine.
+    const bool padded = dims_padded(d);
+    auto fast = [&](int which) {
+        const int L = which == 0 || which == 4 ? d.Lx : which == 2 ? d.Lz : d.Ly;
+        const Engine e = engine_of(m, L, padded);
+        return (e == kPow2 && launch_fast<T>(m, which, io)) || (e == kMix && launch_mix<T>(m, which, io));
+    };
 
     // ---- forward x, y ----
     cpx<T> *F = static_cast<cpx<T> *>(io.fwd);
@@ -617,7 +621,8 @@ int ensure_workspace(Mesh *m)
     if (ws.ready) return SC_OK;
     Ctx *ctx = m->ctx;
     const Dims d = make_dims(m);
-    // transform half-lengths (padded beyond the mesh's nodes where 2n is not 7-smooth)
+    ws.smooth = smooth_lengths(m);
+    // transform half-lengths (padded beyond the mesh's nodes, see transform_half)
     const int64_t nx = d.nx, ny = d.ny, nz = d.nz;
     const int L[3] = {d.Lx, d.Ly, d.Lz};
     const int64_t mn[3] = {m->n[0], m->n[1], m->n[2]};
@@ -712,8 +717,6 @@ __global__ void __launch_bounds__(256) k_sgroup_store(SStore s, SBunch *__restri
     for (int i = threadIdx.x; i < s.count * kWords; i += blockDim.x) dst[i] = src[i];
 }
 
-bool reg_length(int L) { return L == 32 || L == 64 || L == 128 || L == 256 || L == 512; }
-
 template <typename T>
 int solve_class_t(Ctx *ctx, Mesh *const *ms, int k, const double *const *lo, const double *const *hi,
                   const double *const *dl, const double *gamma, int cath, SBunch *tab)
@@ -760,7 +763,11 @@ int solve_class_t(Ctx *ctx, Mesh *const *ms, int k, const double *const *lo, con
     static const int kid[5] = {K_RHO_FWD_X, K_RHO_FWD_Y, K_ZCONV, K_INV_Y, K_INV_X};
     for (int which = 0; which < 5; ++which) {
         launch_begin(ctx, kid[which]);
-        launch_fast_grouped<T>(ms[0], k, tab, which, mode, 1, 3, st);
+        const int L = which == 0 || which == 4 ? d.Lx : which == 2 ? d.Lz : d.Ly;
+        if (engine_of(ms[0], L, dims_padded(d)) == kPow2)
+            launch_fast_grouped<T>(ms[0], k, tab, which, mode, 1, 3, st);
+        else
+            launch_mix_grouped<T>(ms[0], k, tab, which, mode, 1, 3, st);
         launch_end(ctx, kid[which]);
         if (which == 2 && !stream_capturing(st, &cid)) {
             // a later single solve's side-stream Green build waits for this
@@ -782,9 +789,11 @@ int solve_class_t(Ctx *ctx, Mesh *const *ms, int k, const double *const *lo, con
 
 bool solve_groupable(const Mesh *m)
 {
-    if (m->generic_transforms || m->green_reuse) return false;
+    if (m->green_reuse) return false;
     const Dims d = make_dims(m);
-    return !dims_padded(d) && reg_length(d.Lx) && reg_length(d.Ly) && reg_length(d.Lz);
+    const bool padded = dims_padded(d);
+    return engine_of(m, d.Lx, padded) != kGeneric && engine_of(m, d.Ly, padded) != kGeneric &&
+           engine_of(m, d.Lz, padded) != kGeneric;
 }
 
 int64_t solve_group_bytes(const Mesh *m)

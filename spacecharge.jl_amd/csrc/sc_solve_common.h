@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include "sc_fft_dev.h"
+#include "sc_fft_mix.h"
 #include "sc_internal.h"
 
 namespace sc {
@@ -21,20 +22,52 @@ inline bool smooth7(int L)
 }
 
 // Transform half-length of an axis of n nodes: the smallest t >= n whose 2t
-// has no prime factor above 7.  The reference zero-pads each axis to exactly
-// 2n (src/mesh.jl:51-61) and FFTW transforms any length.  The convolution it
-// computes is linear: output node m < n sums rho[j] G(m - j) over j < n, lags
-// |m - j| <= n - 1, so any cyclic length of at least 2n - 1 gives the same
-// outputs.  Axes whose 2n has a larger prime factor are therefore padded
+// the register engines transform (sc_fft_mix.h), on axes beyond those lengths
+// (n > 256) the smallest whose 2t has no prime factor above 7.  The reference
+// zero-pads each axis to exactly 2n (src/mesh.jl:51-61) and FFTW transforms
+// any length.  The convolution it computes is linear: output node m < n sums
+// rho[j] G(m - j) over j < n, lags |m - j| <= n - 1, so any cyclic length of
+// at least 2n - 1 gives the same outputs.  Other axes are therefore padded
 // further, to 2t: rho stays zero beyond its n nodes, the Green function is
 // built on t lags (its first n are the reference's cell integrals; it depends
 // on the spacing, gamma and the image offset only, not on n), and only the n
-// physical outputs are written.  t == n for every axis whose 2n is 7-smooth.
-inline int transform_half(int n)
+// physical outputs are written.  Padding to the next register length beats
+// transforming 2n itself on the generic engine also where the padding is
+// widest (one solve, generic at 2n's own length -> register: 201^3, 402 -> 512
+// points, 2994 -> 1531 us in Float32 and 4748 -> 2584 us in Float64; 101^3,
+// 210 -> 256, 386 -> 162 and 549 -> 269 us; 161^3 Float64 with the cathode,
+// 324 -> 384, 3377 -> 2861 us).
+inline bool reg_length(int L)
+{
+    switch (L) {
+#define X(LL) case LL:
+        SC_MIX_LENGTHS(X)
+#undef X
+        return true;
+    default: return false;
+    }
+}
+
+inline int transform_half(int n, bool smooth)
 {
     int t = n;
+    if (!smooth && 2 * n <= kMixMaxLength) {
+        while (!reg_length(2 * t)) ++t;
+        return t;
+    }
     while (!smooth7(2 * t)) ++t;
     return t;
+}
+
+// Float32 meshes that carry Float64 particles keep the plain 7-smooth lengths
+// (and with them the generic engine, except for unpadded powers of two).
+// Their caller gets the interpolated fields in Float64 and so sees the
+// transforms' Float32 rounding itself, which any other length or radix moves
+// by 1e-7 of the field: such fields stay reproducible to the last bits.  The
+// choice is made when the mesh's workspace is, by the particles deposited so far.
+inline bool smooth_lengths(const Mesh *m)
+{
+    return m->ws.ready ? m->ws.smooth : m->f64_particles && m->dtype == SC_F32;
 }
 
 // Shape of a solve.  nx, ny, nz are the transform half-lengths (the Green
@@ -56,9 +89,10 @@ inline Dims make_dims(const Mesh *m)
     d.mx = (int)m->n[0];
     d.my = (int)m->n[1];
     d.mz = (int)m->n[2];
-    d.nx = transform_half(d.mx);
-    d.ny = transform_half(d.my);
-    d.nz = transform_half(d.mz);
+    const bool smooth = smooth_lengths(m);
+    d.nx = transform_half(d.mx, smooth);
+    d.ny = transform_half(d.my, smooth);
+    d.nz = transform_half(d.mz, smooth);
     d.Kx = d.nx + 1;
     d.Kp = (d.Kx + 31) / 32 * 32;
     d.Lx = 2 * d.nx;
@@ -67,7 +101,18 @@ inline Dims make_dims(const Mesh *m)
     return d;
 }
 
-// true when some axis is padded beyond twice its nodes (generic engine only)
+// Engine of a transform of length L: the power-of-two register engine where no
+// axis is padded (the Green passes work on the padded extents throughout and
+// pass padded = false), else the mixed-radix one, else (longer axes, meshes
+// with smooth_lengths, force_generic_transforms) the generic LDS engine.
+enum Engine { kGeneric, kPow2, kMix };
+inline Engine engine_of(const Mesh *m, int L, bool padded)
+{
+    if (m->generic_transforms || !reg_length(L)) return kGeneric;
+    if (!padded && L >= 32 && (L & (L - 1)) == 0) return kPow2;
+    return smooth_lengths(m) ? kGeneric : kMix;
+}
+// true when some axis is padded beyond twice its nodes
 inline bool dims_padded(const Dims &d) { return d.nx != d.mx || d.ny != d.my || d.nz != d.mz; }
 
 inline int div_up(int a, int b) { return (a + b - 1) / b; }
@@ -157,14 +202,16 @@ template <typename T>
 int build_green(Mesh *m, const double dl[3], double gamma, double offz, int mode);
 
 // Solve kernel `which` (0 forward x, 1 forward y, 2 z convolution, 3 inverse
-// y, 4 inverse x) of `io` on the register-resident engine; false when its
-// transform length is not one of the supported powers of two (nothing is
-// launched then).
+// y, 4 inverse x) of `io` on the power-of-two (launch_fast) or mixed-radix
+// (launch_mix) register engine; false when the engine does not take it
+// (nothing is launched then).
 template <typename T>
 bool launch_fast(Mesh *m, int which, const SolveIO &io);
+template <typename T>
+bool launch_mix(Mesh *m, int which, const SolveIO &io);
 
-// Grouped forms, on `st`, for nb bunches of mesh shape d whose transform
-// lengths are supported powers of two: the Green build (field modes) of
+// Grouped forms, on `st`, for nb bunches of the mesh shape of m0 whose
+// transforms run on the register engines: the Green build (field modes) of
 // every bunch, from m0's twiddles and the table's spacings, and solve
 // kernel `which` of every bunch with the table's buffers.
 template <typename T>
@@ -173,5 +220,8 @@ void build_green_grouped(const Mesh *m0, int nb, const SBunch *tab, double gamma
 template <typename T>
 void launch_fast_grouped(const Mesh *m0, int nb, const SBunch *tab, int which, int mode, int nin,
                          int nout, hipStream_t st);
+template <typename T>
+void launch_mix_grouped(const Mesh *m0, int nb, const SBunch *tab, int which, int mode, int nin,
+                        int nout, hipStream_t st);
 
 }  // namespace sc
