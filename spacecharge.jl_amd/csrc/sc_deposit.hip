@@ -31,6 +31,8 @@
 //   gather_tiles   one lane per node: sum over the (up to 8) tiles whose
 //               sub-grid holds the node, in a fixed order
 //
+// Meshes of few tiles skip the binning (k_deposit_direct, direct_slices).
+//
 // A particle's eight contributions are computed exactly as in the reference
 // (same operation order, no FMA contraction); only the order of the sums
 // differs, and the sums run in Float64.  Meshes with more tiles than one
@@ -60,6 +62,13 @@ constexpr int kBatch = 8;            // particles a lane loads before computing 
 // (Mesh::chunk_log2, kChunkLog2Min..kChunkLog2Max)
 constexpr int kDepThreads = 512;     // deposit workgroup size
 constexpr int kBinMaxSlices = 2048;  // binning workgroups (columns of the count matrix)
+
+// direct deposit (k_deposit_direct): most tiles, most particle-tile pairs (most
+// particles on one tile), particles per workgroup, workgroups aimed at
+constexpr int kDirectTiles = 64;
+constexpr int64_t kDirectPairs = (int64_t)4 << 20, kDirectMost = (int64_t)16 << 20;
+constexpr int kDirectLog2 = 13;
+constexpr int kDirectBlocks = 128;
 
 inline int div_up4(int a) { return (a + 3) / 4; }
 
@@ -624,6 +633,22 @@ __device__ __forceinline__ void deposit_chunk(const Rec<PT> *__restrict__ src,
     }
 }
 
+// Scale of the fixed-point accumulator for contributions of at most qm, at most
+// 2^log2n of them in one sum: false (Float64 instead) unless qm is finite and
+// not so small that the scale 2^(48 - ilogb) overflows.
+__device__ __forceinline__ bool fixed_scale(double qm, int log2n, double &S, double &invS)
+{
+    if (!(qm <= 1.7976931348623157e308 && (qm == 0.0 || qm >= 1e-270))) return false;
+    if (qm > 0.0) {
+        // |q 2^e| < 2^49 (the rounding in deposit_one needs < 2^51) and
+        // 2^log2n * qm * 2^e < 2^62 (no sum overflows)
+        const int e = (log2n <= 13 ? 48 : 61 - log2n) - ilogb(qm);
+        S = ldexp(1.0, e);
+        invS = ldexp(1.0, -e);
+    }
+    return true;
+}
+
 // Grid (chunks, channels): channel c takes its charges from the records
 // (c = 0) or from qs[c - 1] in the records' order, its max|q| from the
 // slice maxima kBinMaxSlices * c in, and writes sub-grid set c (pstride
@@ -662,17 +687,7 @@ __device__ __forceinline__ void deposit_tiles_body(
         m = wmax[0];
         for (int k = 1; k < (int)(blockDim.x >> 6); ++k) m = wmax[k] > m ? wmax[k] : m;
         const double qm = __longlong_as_double((long long)m);
-        // finite max|q| not so small that the scale 2^(48 - ilogb) overflows
-        if (ext_flags[t] == 0u && qm <= 1.7976931348623157e308 && (qm == 0.0 || qm >= 1e-270)) {
-            fixed = true;
-            if (qm > 0.0) {
-                // |q 2^e| < 2^49 (the rounding below needs < 2^51) and
-                // 2^chunk_log2 * qm * 2^e < 2^62 (no sum overflows)
-                const int e = (chunk_log2 <= 13 ? 48 : 61 - chunk_log2) - ilogb(qm);
-                S = ldexp(1.0, e);
-                invS = ldexp(1.0, -e);
-            }
-        }
+        fixed = ext_flags[t] == 0u && fixed_scale(qm, chunk_log2, S, invS);
     }
     for (int i = threadIdx.x; i < kSubVol; i += blockDim.x) sub[i] = 0.0;  // also integer zero
     __syncthreads();
@@ -806,6 +821,299 @@ k_gather_tiles(const double *__restrict__ partials, size_t pstride,
                           chan == 0 ? rho0 : (chan == 1 ? rho1 : rho2), accumulate, skip_empty);
 }
 
+// ---- deposit without binning: meshes of few tiles ----
+// The binned chain is six dependent launches, 27-40 us however few the
+// particles (and 22 us of the host's time).  On a mesh of few tiles a workgroup per (particle slice, tile)
+// reads its slice and deposits the particles of its tile straight into the
+// tile's LDS sub-grid, in the same arithmetic, and a node-parallel sum over
+// tiles and slices follows: two launches (three for Float32 meshes), no
+// records, no tile tables.  Bound by its dependent phases (read, list, deposit,
+// store) and by the 39 KB sub-grid that each workgroup writes.  The
+// particles are read once per tile (from the L2), so the product of tiles and
+// particles bounds the range (direct_slices).
+//
+// Float32 meshes accumulate in fixed point by the binned chain's rules (the
+// scale from max|q| over all particles, Float64 in tiles that hold a particle
+// with weights outside [0, 1]), so that both give the same bits; a launch
+// before it (k_direct_prep) finds the two.
+
+// max|q| of each channel and the mask of tiles that hold an extrapolating
+// particle, per slice of the particles (workgroup w: qmax[c * kBinMaxSlices +
+// w], ext[w]).
+template <typename PT, typename MT, int NCH>
+__global__ void __launch_bounds__(kBinThreads)
+k_direct_prep(const PT *__restrict__ px, const PT *__restrict__ py, const PT *__restrict__ pz,
+              const PT *__restrict__ q0, const PT *__restrict__ q1, const PT *__restrict__ q2, Split sp,
+              Geo g, unsigned long long *__restrict__ ext, unsigned long long *__restrict__ qmax)
+{
+    resolve_geo(g);
+    __shared__ unsigned long long wred[NCH + 1][kBinThreads / 64];
+    const PT *pq[3] = {q0, q1, q2};
+    const int64_t first = (int64_t)blockIdx.x * sp.slice;
+    const int64_t end = first + sp.slice < sp.n ? first + sp.slice : sp.n;
+    double qm[NCH] = {};
+    unsigned long long mask = 0ull;
+    for (int64_t base = first; base < end; base += kBatch * kBinThreads) {
+        PT x[kBatch], y[kBatch], z[kBatch], q[NCH][kBatch];
+#pragma unroll
+        for (int s = 0; s < kBatch; ++s) {
+            int64_t p = base + s * kBinThreads + threadIdx.x;
+            p = p < end ? p : end - 1;  // a repeated particle changes neither result
+            x[s] = px[p];
+            y[s] = py[p];
+            z[s] = pz[p];
+#pragma unroll
+            for (int c = 0; c < NCH; ++c) q[c][s] = pq[c][p];
+        }
+#pragma unroll
+        for (int s = 0; s < kBatch; ++s) {
+            bool e;
+            const int t = tile_of<PT, MT>(x[s], y[s], z[s], g, e);
+            mask |= e ? 1ull << t : 0ull;
+#pragma unroll
+            for (int c = 0; c < NCH; ++c) {
+                const double aq = fabs((double)q[c][s]);
+                qm[c] = (aq > qm[c] || aq != aq) ? aq : qm[c];  // NaN sticks
+            }
+        }
+    }
+#pragma unroll
+    for (int c = 0; c <= NCH; ++c) {
+        // |q| >= 0: its bit pattern orders like its value (NaN above +inf)
+        unsigned long long v = c < NCH ? (unsigned long long)__double_as_longlong(qm[c < NCH ? c : 0]) : mask;
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) {
+            const unsigned long long o = __shfl_xor(v, d, 64);
+            v = c < NCH ? (o > v ? o : v) : (v | o);
+        }
+        if ((threadIdx.x & 63) == 0) wred[c][threadIdx.x >> 6] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x <= NCH) {
+        const int c = threadIdx.x;
+        unsigned long long v = wred[c][0];
+        for (int k = 1; k < kBinThreads / 64; ++k) {
+            const unsigned long long o = wred[c][k];
+            v = c < NCH ? (o > v ? o : v) : (v | o);
+        }
+        if (c < NCH) qmax[(size_t)c * kBinMaxSlices + blockIdx.x] = v;
+        else ext[blockIdx.x] = v;
+    }
+}
+
+// Grid (slices, tiles, channels).  On a mesh of several tiles a first pass over
+// the slice lists the particles of the tile (16-bit offsets in LDS, so that the
+// deposit runs with full waves); the deposit of the listed particles follows.
+// used[tile][slice] is 0 where the slice has no particle in the tile; the
+// sub-grid is then unset.  W: workgroups of k_direct_prep (Float32 meshes).
+template <typename PT, typename MT>
+__global__ void __launch_bounds__(kDepThreads)
+k_deposit_direct(const PT *__restrict__ px, const PT *__restrict__ py, const PT *__restrict__ pz,
+                 const PT *__restrict__ q0, const PT *__restrict__ q1, const PT *__restrict__ q2,
+                 Split sp, Geo g, double *__restrict__ partials, size_t pstride,
+                 unsigned *__restrict__ used, const unsigned long long *__restrict__ ext,
+                 const unsigned long long *__restrict__ qmax, int W)
+{
+    resolve_geo(g);
+    __shared__ double sub[kSubVol];
+    __shared__ unsigned short list[1 << kDirectLog2];
+    __shared__ unsigned long long wred[2][kDepThreads / 64];
+    __shared__ int s_count;
+    const int t = blockIdx.y, chan = blockIdx.z;
+    const bool one = gridDim.y == 1;
+    const int lane = threadIdx.x & 63;
+    const PT *pq = chan == 0 ? q0 : (chan == 1 ? q1 : q2);
+    const int64_t first = (int64_t)blockIdx.x * sp.slice;
+    const int len = (int)((first + sp.slice < sp.n ? first + sp.slice : sp.n) - first);
+    px += first;
+    py += first;
+    pz += first;
+    pq += first;
+    if constexpr (sizeof(MT) == 4) {
+        unsigned long long m = 0ull, e = 0ull;
+        for (int i = threadIdx.x; i < W; i += kDepThreads) {
+            const unsigned long long o = qmax[(size_t)chan * kBinMaxSlices + i];
+            m = o > m ? o : m;
+            e |= ext[i];
+        }
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) {
+            const unsigned long long o = __shfl_xor(m, d, 64);
+            m = o > m ? o : m;
+            e |= __shfl_xor(e, d, 64);
+        }
+        if (lane == 0) {
+            wred[0][threadIdx.x >> 6] = m;
+            wred[1][threadIdx.x >> 6] = e;
+        }
+    }
+    for (int i = threadIdx.x; i < kSubVol; i += kDepThreads) sub[i] = 0.0;  // also integer zero
+    if (threadIdx.x == 0) s_count = 0;
+    __syncthreads();
+    if (!one) {
+        for (int base = 0; base < len; base += kBatch * kDepThreads) {
+            PT x[kBatch], y[kBatch], z[kBatch];
+#pragma unroll
+            for (int s = 0; s < kBatch; ++s) {
+                int p = base + s * kDepThreads + (int)threadIdx.x;
+                p = p < len ? p : len - 1;  // unconditional loads stay in flight together
+                x[s] = px[p];
+                y[s] = py[p];
+                z[s] = pz[p];
+            }
+            bool mine[kBatch];
+            int before[kBatch], total = 0;
+#pragma unroll
+            for (int s = 0; s < kBatch; ++s) {
+                mine[s] = tile_of<PT, MT>(x[s], y[s], z[s], g) == t &&
+                          base + s * kDepThreads + (int)threadIdx.x < len;
+                const unsigned long long b = __ballot(mine[s]);
+                before[s] = total + __popcll(b & ((1ull << lane) - 1ull));
+                total += __popcll(b);
+            }
+            if (total) {  // uniform over the wave
+                int at = 0;
+                if (lane == 0) at = atomicAdd(&s_count, total);
+                at = __shfl(at, 0, 64);
+#pragma unroll
+                for (int s = 0; s < kBatch; ++s)
+                    if (mine[s])
+                        list[at + before[s]] = (unsigned short)(base + s * kDepThreads + (int)threadIdx.x);
+            }
+        }
+        __syncthreads();
+    }
+    const int count = one ? len : s_count;
+    const size_t slot = (size_t)t * sp.G + blockIdx.x;
+    if (threadIdx.x == 0) used[(size_t)chan * gridDim.y * sp.G + slot] = (unsigned)count;
+    if (count == 0) return;  // uniform over the workgroup
+    bool fixed = false;
+    double S = 1.0, invS = 1.0;
+    if constexpr (sizeof(MT) == 4) {
+        unsigned long long m = wred[0][0], e = wred[1][0];
+        for (int k = 1; k < kDepThreads / 64; ++k) {
+            m = wred[0][k] > m ? wred[0][k] : m;
+            e |= wred[1][k];
+        }
+        fixed = !((e >> t) & 1ull) && fixed_scale(__longlong_as_double((long long)m), kDirectLog2, S, invS);
+    }
+    const int ox = (t % g.tx) * kTile, oy = ((t / g.tx) % g.ty) * kTile, oz = (t / (g.tx * g.ty)) * kTile;
+    constexpr int kB = 4;  // particles whose loads are in flight together
+    for (int i0 = 0; i0 < count; i0 += kB * kDepThreads) {
+        Rec<PT> r[kB];
+#pragma unroll
+        for (int u = 0; u < kB; ++u) {
+            int i = i0 + u * kDepThreads + (int)threadIdx.x;
+            i = i < count ? i : count - 1;
+            const int p = one ? i : (int)list[i];
+            r[u].x = px[p];
+            r[u].y = py[p];
+            r[u].z = pz[p];
+            r[u].q = pq[p];
+        }
+#pragma unroll
+        for (int u = 0; u < kB; ++u) {
+            if (i0 + u * kDepThreads + (int)threadIdx.x < count) {
+                if (fixed) deposit_one<PT, MT, true>(r[u], g, ox, oy, oz, sub, S);
+                else deposit_one<PT, MT, false>(r[u], g, ox, oy, oz, sub, S);
+            }
+        }
+    }
+    __syncthreads();
+    double *out = partials + chan * pstride + slot * kSubVol;
+    if (fixed) {
+        const long long *si = reinterpret_cast<const long long *>(sub);
+        for (int i = threadIdx.x; i < kSubVol; i += kDepThreads) out[i] = (double)si[i] * invS;
+    } else {
+        for (int i = threadIdx.x; i < kSubVol; i += kDepThreads) out[i] = sub[i];
+    }
+}
+
+// rho from the direct deposit's sub-grids: per node, the sum over the (up to
+// 8) tiles that hold it and the G slices.  A workgroup takes 256 / SL nodes
+// with SL lanes each, which share the slices and add up through LDS, in a
+// fixed order.  Grid (node blocks, channels).
+template <typename MT, int SL>
+__global__ void __launch_bounds__(256)
+k_gather_direct(const double *__restrict__ partials, size_t pstride, const unsigned *__restrict__ used,
+                int G, Geo g, MT *__restrict__ rho0, MT *__restrict__ rho1, MT *__restrict__ rho2,
+                int accumulate)
+{
+    constexpr int NN = 256 / SL;  // nodes of the workgroup
+    __shared__ double part[SL][NN];
+    const int chan = blockIdx.y, T = g.tx * g.ty * g.tz;
+    partials += chan * pstride;
+    used += (size_t)chan * T * G;
+    const int M = g.nx * g.ny * g.nz;
+    const int ln = threadIdx.x % NN, s0 = threadIdx.x / NN;
+    const int i = (int)blockIdx.x * NN + ln;
+    double s = 0.0;
+    if (i < M) {
+        const int gx = i % g.nx, gy = (i / g.nx) % g.ny, gz = i / (g.nx * g.ny);
+        // along an axis: the tile that starts at or before the node, and the one
+        // before it when the node is on their face
+        const int ax = gx / kTile, ay = gy / kTile, az = gz / kTile;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            const int cx = ax - (c & 1), cy = ay - ((c >> 1) & 1), cz = az - (c >> 2);
+            const int lx = gx - kTile * cx, ly = gy - kTile * cy, lz = gz - kTile * cz;
+            if (cx < 0 || cy < 0 || cz < 0 || cx >= g.tx || cy >= g.ty || cz >= g.tz || lx > kTile ||
+                ly > kTile || lz > kTile)
+                continue;
+            const size_t slot = (size_t)(cx + g.tx * (cy + g.ty * cz)) * G;
+            const double *p = partials + slot * kSubVol + lx + kSub * (ly + kSub * lz);
+            // U slices' loads in flight together; an unset sub-grid is read
+            // beside its flag and not added
+            constexpr int U = SL == 1 ? 1 : SL == 4 ? 2 : 4;
+            for (int k0 = s0; k0 < G; k0 += U * SL) {
+                unsigned on[U];
+                double v[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int k = k0 + u * SL < G ? k0 + u * SL : G - 1;
+                    on[u] = used[slot + k];
+                    v[u] = p[(size_t)k * kSubVol];
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u) s += (on[u] != 0u && k0 + u * SL < G) ? v[u] : 0.0;
+            }
+        }
+    }
+    part[s0][ln] = s;
+    __syncthreads();
+    if (s0 == 0 && i < M) {
+        double a = part[0][ln];
+#pragma unroll
+        for (int k = 1; k < SL; ++k) a += part[k][ln];
+        MT *rho = chan == 0 ? rho0 : (chan == 1 ? rho1 : rho2);
+        rho[i] = accumulate ? (MT)((double)rho[i] + a) : (MT)a;
+    }
+}
+
+// Slices of the direct deposit (nchan charge channels) of n particles on a mesh
+// of T tiles, or 0 where the binned chain takes it: a mesh with a deposit
+// tiling of its own, and too many particle-tile pairs.  Measured (replayed from
+// a graph, direct / binned, us), Float64: 10k particles on 16^3 7.7 / 37; 50k
+// and 200k on 32^3 (8 tiles) 19 / 38 and 27 / 43, 1M 86 / 54; 50k on 64^3 (64
+// tiles) 34 / 39, 200k 76 / 44: the two cross near 4M pairs.  Float32, with one
+// launch more: 10k on 16^3 13 / 32, 1M 25 / 50; 200k on 32^3 29 / 40; 50k on 48^3
+// (27 tiles) 37 / 35: near 1.5M pairs, kept at 2M for the three launches that it
+// saves the host.  One tile has no pairs to spare: there only the size of the
+// sub-grids ends the range.
+int direct_slices(const Mesh *m, int64_t n, int T, int nchan)
+{
+    if (m->chunk_log2 != kChunkLog2Default || m->slice_log2 != kSliceLog2Default) return 0;
+    const int64_t most_pairs = T == 1 ? kDirectMost : (m->dtype == SC_F32 ? kDirectPairs / 2 : kDirectPairs);
+    if (T > kDirectTiles || n * T * nchan > most_pairs) return 0;
+    const int64_t per = (int64_t)1 << kDirectLog2;
+    const int64_t least = (n + per - 1) / per;  // slices of at most 2^kDirectLog2
+    const int64_t most = (n + kDepThreads - 1) / kDepThreads;
+    int64_t G = (T == 1 ? 2 : 1) * kDirectBlocks / T;
+    if (G > most) G = most;
+    if (G < least) G = least;
+    return (int)G;
+}
+
 // At most kBinMaxSlices slices of about 2^slice_log2 particles, and at
 // most kCmatBudget / ntiles (the count matrix has a row per tile).
 Split split_of(int64_t n, int slice_log2, int ntiles)
@@ -828,6 +1136,44 @@ Split split_of(int64_t n, int slice_log2, int ntiles)
 // binning range (the layout the grouped launches assume), else the tiles.
 int counts_stride(int ntiles) { return ntiles > kRange ? ntiles : kRange; }
 
+// Room for `need` chunks and sub-grids in each of nchan channel sets.
+int grow_partials(Mesh *m, int64_t need, int nchan)
+{
+    DepositBins &B = m->bins;
+    auto fail = [&]() {
+        return set_err(m->ctx, SC_ERR_NOMEM, "device allocation of the deposit bins failed");
+    };
+    const int64_t cap = B.chunk_cap > need ? B.chunk_cap : need;
+    const int sets = B.partial_sets > nchan ? B.partial_sets : nchan;
+    if (B.chunks) (void)hipFree(B.chunks);
+    if (B.partials) (void)hipFree(B.partials);
+    B.chunks = B.partials = nullptr;
+    B.chunk_cap = 0;
+    B.partial_sets = 0;
+    if (hipMalloc(&B.chunks, sizeof(int4) * cap) != hipSuccess) return fail();
+    // one sub-grid per chunk and channel, in the wider mesh type (double
+    // covers both); channel c's set starts c * cap sub-grids in
+    if (hipMalloc(&B.partials, sizeof(double) * kSubVol * (size_t)cap * sets) != hipSuccess)
+        return fail();
+    B.chunk_cap = cap;
+    B.partial_sets = sets;
+    return SC_OK;
+}
+
+int ensure_counts(Mesh *m, int ntiles)
+{
+    DepositBins &B = m->bins;
+    if (B.counts) return SC_OK;
+    // totals | tile start | first extra sub-grid slot | extrapolation flags | nchunks, pad |
+    // per-slice max|q| of up to three channels (u64 bit patterns); the direct
+    // deposit keeps its per-slice tile masks in the first blocks
+    const size_t bytes =
+        sizeof(unsigned) * (4 * (size_t)counts_stride(ntiles) + 4 + 3 * 2 * kBinMaxSlices);
+    if (hipMalloc((void **)&B.counts, bytes) != hipSuccess)
+        return set_err(m->ctx, SC_ERR_NOMEM, "device allocation of the deposit bins failed");
+    return SC_OK;
+}
+
 int ensure_bins(Mesh *m, int64_t n, int pdt, int ntiles, int nchan)
 {
     const int64_t chunk = (int64_t)1 << m->chunk_log2;
@@ -848,28 +1194,9 @@ int ensure_bins(Mesh *m, int64_t n, int pdt, int ntiles, int nchan)
     // (slots of the row scan's reservation order, k_bin_rowscan)
     const int64_t maxchunks = 2 * (int64_t)ntiles + n / chunk + 1;
     if (B.chunk_cap < maxchunks || B.partial_sets < nchan) {
-        const int64_t cap = B.chunk_cap > maxchunks ? B.chunk_cap : maxchunks;
-        const int sets = B.partial_sets > nchan ? B.partial_sets : nchan;
-        if (B.chunks) (void)hipFree(B.chunks);
-        if (B.partials) (void)hipFree(B.partials);
-        B.chunks = B.partials = nullptr;
-        B.chunk_cap = 0;
-        B.partial_sets = 0;
-        if (hipMalloc(&B.chunks, sizeof(int4) * cap) != hipSuccess) return fail();
-        // one sub-grid per chunk and channel, in the wider mesh type (double
-        // covers both); channel c's set starts c * cap sub-grids in
-        if (hipMalloc(&B.partials, sizeof(double) * kSubVol * (size_t)cap * sets) != hipSuccess)
-            return fail();
-        B.chunk_cap = cap;
-        B.partial_sets = sets;
+        if (int rc = grow_partials(m, maxchunks, nchan)) return rc;
     }
-    if (!B.counts) {
-        // totals | tile start | first extra sub-grid slot | extrapolation flags | nchunks, pad |
-        // per-slice max|q| of up to three channels (u64 bit patterns)
-        const size_t bytes =
-            sizeof(unsigned) * (4 * (size_t)counts_stride(ntiles) + 4 + 3 * 2 * kBinMaxSlices);
-        if (hipMalloc((void **)&B.counts, bytes) != hipSuccess) return fail();
-    }
+    if (int rc = ensure_counts(m, ntiles)) return rc;
     const int64_t need_cmat = (int64_t)ntiles * split_of(n, m->slice_log2, ntiles).G;
     if (B.cmat_cap < need_cmat) {
         if (B.cmat) (void)hipFree(B.cmat);
@@ -879,6 +1206,82 @@ int ensure_bins(Mesh *m, int64_t n, int pdt, int ntiles, int nchan)
             return fail();
         B.cmat_cap = need_cmat;
     }
+    return SC_OK;
+}
+
+// Scratch of the direct deposit: T G sub-grids per channel, and their flags.
+int ensure_direct(Mesh *m, int T, int G, int nchan)
+{
+    DepositBins &B = m->bins;
+    auto fail = [&]() {
+        return set_err(m->ctx, SC_ERR_NOMEM, "device allocation of the deposit bins failed");
+    };
+    if (int rc = ensure_counts(m, T)) return rc;
+    const int64_t need = (int64_t)T * G;
+    if (B.chunk_cap < need || B.partial_sets < nchan) {
+        if (int rc = grow_partials(m, need, nchan)) return rc;
+    }
+    if (B.cmat_cap < need * nchan) {
+        if (B.cmat) (void)hipFree(B.cmat);
+        B.cmat = nullptr;
+        B.cmat_cap = 0;
+        if (hipMalloc((void **)&B.cmat, sizeof(unsigned) * (size_t)(need * nchan)) != hipSuccess)
+            return fail();
+        B.cmat_cap = need * nchan;
+    }
+    return SC_OK;
+}
+
+template <typename PT, typename MT>
+int direct(Mesh *m, const void *x, const void *y, const void *z, const void *const *q, int nchan,
+           int64_t n, const Geo &g, int clear, void *const *out, int G)
+{
+    Ctx *ctx = m->ctx;
+    hipStream_t st = ctx->stream;
+    DepositBins &B = m->bins;
+    const int T = g.tx * g.ty * g.tz;
+    Split sp;
+    sp.n = n;
+    sp.G = G;
+    sp.slice = (n + G - 1) / G;
+    const size_t pstride = (size_t)kSubVol * (size_t)B.chunk_cap;
+    const PT *px = (const PT *)x, *py = (const PT *)y, *pz = (const PT *)z, *q0 = (const PT *)q[0];
+    const PT *q1 = (const PT *)q[nchan > 1 ? 1 : 0], *q2 = (const PT *)q[nchan > 2 ? 2 : 0];
+    auto *ext = reinterpret_cast<unsigned long long *>(B.counts);
+    auto *qmax = reinterpret_cast<unsigned long long *>(B.counts + 4 * counts_stride(T) + 4);
+    Split pre = sp;  // of k_direct_prep: at most kBinMaxSlices slices (kRange u64 masks fit)
+    if (sizeof(MT) == 4) {
+        const int64_t most = (n + kBatch * kBinThreads - 1) / (kBatch * kBinThreads);
+        pre.G = (int)(most < kBinMaxSlices ? most : kBinMaxSlices);
+        pre.slice = (n + pre.G - 1) / pre.G;
+        launch_begin(ctx, K_BIN_COUNT);
+        auto prep = nchan == 3 ? k_direct_prep<PT, MT, 3> : k_direct_prep<PT, MT, 1>;
+        hipLaunchKernelGGL(prep, dim3(pre.G), dim3(kBinThreads), 0, st, px, py, pz, q0, q1, q2, pre, g,
+                           ext, qmax);
+        launch_end(ctx, K_BIN_COUNT);
+    }
+    launch_begin(ctx, K_DEPOSIT_TILES);
+    hipLaunchKernelGGL((k_deposit_direct<PT, MT>), dim3(G, T, nchan), dim3(kDepThreads), 0, st,
+                       px, py, pz, q0, q1, q2, sp, g, static_cast<double *>(B.partials), pstride,
+                       B.cmat, (const unsigned long long *)ext, (const unsigned long long *)qmax, pre.G);
+    launch_end(ctx, K_DEPOSIT_TILES);
+    MT *o0 = static_cast<MT *>(out[0]);
+    MT *o1 = nchan > 1 ? static_cast<MT *>(out[1]) : o0;
+    MT *o2 = nchan > 2 ? static_cast<MT *>(out[2]) : o0;
+    const int64_t M = (int64_t)g.nx * g.ny * g.nz;
+    launch_begin(ctx, K_GATHER_TILES);
+    auto gather = [&](auto slc) {
+        constexpr int SL = decltype(slc)::value;
+        hipLaunchKernelGGL((k_gather_direct<MT, SL>), dim3((unsigned)((M * SL + 255) / 256), nchan),
+                           dim3(256), 0, st, (const double *)B.partials, pstride,
+                           (const unsigned *)B.cmat, G, g, o0, o1, o2, clear ? 0 : 1);
+    };
+    if (G >= 64) gather(std::integral_constant<int, 16>{});
+    else if (G >= 8) gather(std::integral_constant<int, 8>{});
+    else if (G >= 2) gather(std::integral_constant<int, 4>{});
+    else gather(std::integral_constant<int, 1>{});
+    launch_end(ctx, K_GATHER_TILES);
+    SC_HIP(ctx, hipGetLastError());
     return SC_OK;
 }
 
@@ -1068,8 +1471,19 @@ int launch_deposit_binned_multi(Mesh *m, int pdt, const void *x, const void *y, 
         g.lo[a] = lo ? lo[a] : 0.0;
         g.dl[a] = lo ? dl[a] : 1.0;
     }
-    if (int rc = ensure_bins(m, n, pdt, g.tx * g.ty * g.tz, nchan)) return rc;
     note_particles(m, pdt);
+    const int T = g.tx * g.ty * g.tz;
+    if (const int G = direct_slices(m, n, T, nchan)) {
+        if (int rc = ensure_direct(m, T, G, nchan)) return rc;
+        if (pdt == SC_F32 && m->dtype == SC_F32)
+            return direct<float, float>(m, x, y, z, q, nchan, n, g, clear, out, G);
+        if (pdt == SC_F64 && m->dtype == SC_F64)
+            return direct<double, double>(m, x, y, z, q, nchan, n, g, clear, out, G);
+        if (pdt == SC_F64 && m->dtype == SC_F32)
+            return direct<double, float>(m, x, y, z, q, nchan, n, g, clear, out, G);
+        return direct<float, double>(m, x, y, z, q, nchan, n, g, clear, out, G);
+    }
+    if (int rc = ensure_bins(m, n, pdt, T, nchan)) return rc;
     if (nchan > 1) {
         DepositBins &B = m->bins;
         const size_t need = (size_t)2 * n * pdt;

@@ -154,6 +154,8 @@ struct Ctx {
     void *stable = nullptr;
 };
 
+constexpr int kChunkLog2Default = 13, kSliceLog2Default = 12;
+
 // Device workspace of one mesh (lazy, like src/mesh.jl:49-72).
 struct Workspace {
     bool ready = false;
@@ -243,8 +245,8 @@ struct Mesh {
     // (kChunkLog2Min..kChunkLog2Max) and about 2^slice_log2 particles per
     // binning workgroup (kSliceLog2Min..kSliceLog2Max); set by hand or by
     // the autotuner (sc_mesh_autotune_deposit)
-    int chunk_log2 = 13;
-    int slice_log2 = 12;
+    int chunk_log2 = kChunkLog2Default;
+    int slice_log2 = kSliceLog2Default;
 };
 
 // Remembers the widest particles deposited on a Float32 mesh (the lengths of
