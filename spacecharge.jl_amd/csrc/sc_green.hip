@@ -1072,6 +1072,156 @@ k_green_3m(const T *__restrict__ R, T *__restrict__ Gf, cpx<T> *__restrict__ Gi,
     }
 }
 
+// ---- F, the 8-point difference and the x pass in one kernel (field modes) ----
+// k_green_f3 writes 3 (n+1)^3 Float64 values and green_1 reads each of them
+// several times, only to difference them.  Here a workgroup marches along z
+// over the nodes of S y-cell rows: it evaluates the three components of one
+// node plane of its S + 1 node rows into LDS, forms the x differences, keeps
+// those of the plane before in registers, and so holds the cell integrals
+// (differences along x, then z, then y, as diff8v) of S rows, which go through
+// the x transform in place.  The node rows that neighbouring workgroups share
+// are evaluated twice (1/S more, and 1/K more along z for K planes).
+// The values are k_green_f3's: the same terms in the same order; the column
+// and row logs of a plane come from LDS tables, as does log(u^2 + v^2) of each
+// node (one node at a time per lane: with a lane's nodes unrolled the kernel
+// took 238 VGPRs instead of 192 at 256 points and the 128^3 build 79 us, not 75).
+template <typename T, int L>
+struct FxShape {
+    static constexpr int E = Shape<T, L>::E, TPP = Shape<T, L>::TPP;
+    static constexpr int S = L >= 96 ? 8 : 4;           // y cell rows
+    static constexpr int NP = 3 * S / 2;                // pencils: components x row pairs
+    static constexpr int FFT = NP * TPP;                // lanes of the transforms
+    static constexpr int THREADS = FFT <= 256 ? 256 : FFT;
+    static constexpr int NXN = L / 2 + 1, ROWS = S + 1, NODES = ROWS * NXN;
+    static constexpr int M = (NODES + THREADS - 1) / THREADS;  // nodes per lane
+    static constexpr int SLICE = reg::padded<L, E>();
+    static constexpr size_t F_BYTES = sizeof(double) * 3 * NODES;
+    static constexpr size_t T_BYTES = sizeof(cpx<T>) * (NP + 1) * SLICE;  // one slice for idle lanes
+    static constexpr size_t BYTES = F_BYTES > T_BYTES ? F_BYTES : T_BYTES;
+};
+
+template <typename T, int L>
+__global__ void __launch_bounds__((FxShape<T, L>::THREADS))
+k_green_fx(T *__restrict__ R, const cpx<T> *__restrict__ twg, GreenArgs a, int strips, int K,
+           const SBunch *__restrict__ tab, int per)
+{
+    using X = FxShape<T, L>;
+    constexpr int E = X::E, TPP = X::TPP, S = X::S, TH = X::THREADS, NXN = X::NXN;
+    constexpr bool FAST = sizeof(T) == 4;
+    __shared__ cpx<T> tw[L];
+    __shared__ __align__(16) unsigned char shared_[X::BYTES];  // F planes, then the pencils' slices
+    __shared__ double qvw_t[2][X::ROWS], qwu_t[2][NXN], Quv[X::NODES];
+    double *Fs = reinterpret_cast<double *>(shared_);
+    const SBunch *sb;
+    const int bx = group_block(tab, per, sb);
+    if (sb) {
+        R = static_cast<T *>(sb->R);
+        green_from_table(a, sb);
+    }
+    for (int i = threadIdx.x; i < L; i += TH) tw[i] = gld(twg + i);
+    const int image = blockIdx.y, ny = a.d.ny, Kp = a.d.Kp, zc = z_cells(a, image);
+    const int y0 = (bx % strips) * S, k0 = (bx / strips) * K;
+    const int k1 = k0 + K < zc ? k0 + K : zc;  // cells k0 .. k1 - 1, node planes k0 .. k1
+    double dx, dy, dz, offzg;
+    green_geometry(a, dx, dy, dz, offzg);
+    auto coord_u = [&](int i) { return ((double)i - 0.5) * dx; };
+    auto coord_v = [&](int j) { return ((double)(j < ny ? j : ny) - 0.5) * dy; };
+    auto coord_w = [&](int k) {
+        return image ? ((double)(k - a.d.nz) + 0.5) * dz + offzg : ((double)k - 0.5) * dz;
+    };
+    auto tables = [&](int k) {
+        const double w = coord_w(k), ww = w * w;
+        for (int t = threadIdx.x; t < X::ROWS + NXN; t += TH) {
+            const double s = t < NXN ? coord_u(t) : coord_v(y0 + t - NXN);
+            const double q = log_<FAST>(ww + s * s);
+            if (t < NXN) qwu_t[k & 1][t] = q;
+            else qvw_t[k & 1][t - NXN] = q;
+        }
+    };
+    // read back by the lane that writes it
+    for (int n = threadIdx.x; n < X::NODES; n += TH) {
+        const double u = coord_u(n % NXN), v = coord_v(y0 + n / NXN);
+        Quv[n] = log_<FAST>(u * u + v * v);
+    }
+    tables(k0);
+    // this lane's pencil: component c, rows y0 + 2 pair and the next
+    const int p = (int)threadIdx.x / TPP < X::NP ? (int)threadIdx.x / TPP : X::NP;
+    const int j = (int)threadIdx.x % TPP;
+    const int c = p / (S / 2), r0 = 2 * (p % (S / 2)), ya = y0 + r0;
+    const bool live = p < X::NP && ya < ny, hasb = ya + 1 < ny;
+    const T sgn = (c == 0) ? (T)-1 : (T)1;
+    cpx<T> *row = reinterpret_cast<cpx<T> *>(shared_) + p * X::SLICE;
+    const double *Fc = Fs + (p < X::NP ? c * X::NODES + r0 * NXN : 0);
+    double prev[3][E / 2];
+    __syncthreads();
+    for (int kn = k0; kn <= k1; ++kn) {
+        const double w = coord_w(kn), ww = w * w;
+#pragma unroll 1
+        for (int n = threadIdx.x; n < X::NODES; n += TH) {
+            {
+                const int i = n % NXN, rw = n / NXN;
+                const double u = coord_u(i), v = coord_v(y0 + rw);
+                const double uu = u * u, vv = v * v;
+                const double r = sqrt((uu + vv) + ww);
+                const double Lu = log_<FAST>(r + u), Lv = log_<FAST>(r + v), Lw = log_<FAST>(r + w);
+                const double ax = atan_q<FAST>(v * w, r * u);
+                const double ay = atan_q<FAST>(w * u, r * v);
+                const double hp = w == 0.0 ? 0.0
+                                           : ((signbit(u) != signbit(v)) != signbit(w)
+                                                  ? -1.5707963267948966
+                                                  : 1.5707963267948966);
+                const double az = (hp - ax) - ay;
+                Fs[n] = (u * ax - w * Lv) + (v * (Quv[n] - 2.0 * Lw)) * 0.5;
+                Fs[X::NODES + n] = (v * ay - u * Lw) + (w * (qvw_t[kn & 1][rw] - 2.0 * Lu)) * 0.5;
+                Fs[2 * X::NODES + n] = (w * az - v * Lu) + (u * (qwu_t[kn & 1][i] - 2.0 * Lv)) * 0.5;
+            }
+        }
+        __syncthreads();
+        if (kn < k1) tables(kn + 1);  // read after the barriers below
+        cpx<T> v[E];
+#pragma unroll
+        for (int r = 0; r < E / 2; ++r) {
+            const int e = j + r * TPP;
+            double g[3];
+#pragma unroll
+            for (int y = 0; y < 3; ++y) g[y] = Fc[y * NXN + e + 1] - Fc[y * NXN + e];
+            // (x difference at the upper plane minus the lower) at y + 1 minus that at y
+            const double ga = (g[1] - prev[1][r]) - (g[0] - prev[0][r]);
+            const double gb = (g[2] - prev[2][r]) - (g[1] - prev[1][r]);
+            v[r].x = (T)ga;
+            v[r].y = hasb ? (T)gb : (T)0;
+#pragma unroll
+            for (int y = 0; y < 3; ++y) prev[y][r] = g[y];
+        }
+        __syncthreads();  // every lane has read the planes; the slices take their place
+        if (kn == k0) continue;  // uniform: the first plane has none before it
+#pragma unroll
+        for (int r = 0; r < E / 2; ++r) row[j + r * TPP] = v[r];
+        __syncthreads();
+#pragma unroll
+        for (int r = E / 2; r < E; ++r) {
+            const int e = j + r * TPP;
+            const cpx<T> m = row[L - e];  // e >= L / 2; e == L / 2 reads an unused slot
+            v[r] = e == L / 2 ? cpx<T>{(T)0, (T)0} : cpx<T>{sgn * m.x, sgn * m.y};
+        }
+        mix::fft<T, L, E, -1>(v, j, row, 1, tw);
+        if (live) {
+            gbl<T> *Ra = (gbl<T> *)(R + r_off(a, 3 * image + c)) + ((size_t)(kn - 1) * (ny + 1) + ya) * Kp;
+#pragma unroll
+            for (int r = 0; r <= E / 2; ++r) {
+                const int kx = j + r * TPP;
+                if (r < E / 2 || kx == L / 2) {
+                    T ra, rb;
+                    unpack_pair(v[r], c == 0, ra, rb);
+                    Ra[kx] = ra;
+                    if (hasb) Ra[Kp + kx] = rb;
+                }
+            }
+        }
+        __syncthreads();  // the slices are read; the next plane overwrites them
+    }
+}
+
 template <typename T, int L>
 void green_pass_r(int pass, dim3 grid, hipStream_t st, const Workspace &ws, const GreenArgs &a,
                   const cpx<T> *tw)
@@ -1104,6 +1254,52 @@ void green_pass_m(int pass, dim3 grid, hipStream_t st, const Workspace &ws, cons
         hipLaunchKernelGGL((k_green_3m<T, L>), grid, block, 0, st, (const T *)R,
                            static_cast<T *>(ws.Gf), static_cast<cpx<T> *>(ws.Gi), tw, a,
                            (const SBunch *)nullptr, 0);
+}
+
+constexpr int kFxBlocks = 512;
+
+// Whether the fused kernel builds a mesh's Green function.  It is one launch
+// and one pass over F fewer, but evaluates F up to twice (rows and planes at
+// the workgroups' edges) with fewer waves in flight.  Small builds gain (the
+// build of 16^3 Float32 21 -> 13 us, of 32^3 Float64 19 -> 14; the step of 100k
+// particles on 32^3 73 -> 68), and so do those whose F outgrows the 256 MB
+// last-level cache (8M particles on 256^3 Float32 2607 -> 2548 us; 256^3 Float64
+// build 1027 -> 930).  Between, beside the deposit, its longer arithmetic costs
+// more than the traffic it saves (128^3: 401 -> 408 us Float32, 688 -> 696 Float64;
+// 100^3 207 -> 210).  Meshes with smooth_lengths keep the separate kernels' bits.
+bool green_fused(const Mesh *m, const Dims &d, size_t size, int cath)
+{
+    if (smooth_lengths(m) || engine_of(m, d.Lx, false) == kGeneric) return false;
+    const int64_t nodes = (int64_t)(d.nx + 1) * (d.ny + 1) * (cath ? d.nz + 1 + d.Lz : d.nz + 1);
+    return green_small(d, size, cath) || 24 * nodes > ((int64_t)256 << 20);
+}
+
+template <typename T, int L>
+void launch_green_fx(const Dims &d, int cath, hipStream_t st, T *R, const GreenArgs &a,
+                     const cpx<T> *tw, const SBunch *tab, int nb)
+{
+    using X = FxShape<T, L>;
+    const int zc = cath ? d.Lz - 1 : d.nz, strips = div_up(d.ny, X::S);
+    // z planes per workgroup: as many as leave kFxBlocks workgroups
+    int K = (int)((int64_t)strips * zc * (cath ? 2 : 1) * nb / kFxBlocks);
+    K = K < 1 ? 1 : (K > 16 ? 16 : K);
+    const int per = strips * div_up(zc, K);
+    hipLaunchKernelGGL((k_green_fx<T, L>), dim3((unsigned)(per * nb), cath ? 2 : 1), dim3(X::THREADS), 0,
+                       st, R, tw, a, strips, K, tab, per);
+}
+
+// F, difference and x pass in one launch, for register lengths; false otherwise.
+template <typename T>
+bool green_fx(int L, const Dims &d, int cath, hipStream_t st, T *R, const GreenArgs &a,
+              const cpx<T> *tw, const SBunch *tab, int nb)
+{
+    switch (L) {
+#define X(LL) \
+    case LL: launch_green_fx<T, LL>(d, cath, st, R, a, tw, tab, nb); return true;
+        SC_MIX_LENGTHS(X)
+#undef X
+    default: return false;
+    }
 }
 
 // One register-engine Green pass if its length is supported; false otherwise.
@@ -1176,34 +1372,42 @@ int build_green(Mesh *m, const double dl[3], double gamma, double offz, int mode
     const cpx<T> *twy = static_cast<const cpx<T> *>(ws.twT[1]);
     const cpx<T> *twz = static_cast<const cpx<T> *>(ws.twT[2]);
     T *R = static_cast<T *>(ws.R);
-    {
-        const int plane = (d.nx + 1) * (d.ny + 1);
-        const int znodes = cath ? d.Lz : d.nz + 1;
+    bool fused = false;
+    if (!a.pot && green_fused(m, d, sizeof(T), cath)) {
         launch_begin(ctx, K_GREEN_F);
-        if (!a.pot)
-            hipLaunchKernelGGL(k_green_f3<sizeof(T) == 4>,
-                               dim3((unsigned)div_up(plane, 256), div_up(znodes, kF3Planes), cath ? 2 : 1),
-                               dim3(256), 0, st, ws.F, a, (const SBunch *)nullptr, 0);
-        else
-            hipLaunchKernelGGL(k_green_f<sizeof(T) == 4>,
-                               dim3((unsigned)div_up(plane, 256), znodes, ncomp), dim3(256), 0, st,
-                               ws.F, a, (const SBunch *)nullptr, 0);
+        fused = green_fx<T>(d.Lx, d, cath, st, R, a, twx, nullptr, 1);
         launch_end(ctx, K_GREEN_F);
     }
-    launch_begin(ctx, K_GREEN_X);
-    if (engine_of(m, d.Lx, false) == kGeneric ||
-        !green_pass_fast<T>(1, d.Lx, ncomp, d, cath, st, ws, a, twx)) {
-        with_fft_elems<T>(d.Lx, [&](auto e, auto t) {
-            constexpr int E = decltype(e)::value, NT = decltype(t)::value;
-            const int nb = pick_nb(d.Lx, E * NT, 16);
-            const int zc = cath ? d.Lz - 1 : d.nz;
-            const int np = zc * ((d.ny + 1) / 2);
-            const size_t sh = sizeof(cpx<T>) * (d.Lx + (size_t)nb * d.Lx);
-            hipLaunchKernelGGL((k_green_1<T, E, NT>), dim3(div_up(np, nb), ncomp), dim3(NT), sh,
-                               st, (const double *)ws.F, R, twx, ws.plan[0], a, nb);
-        });
+    if (!fused) {
+        {
+            const int plane = (d.nx + 1) * (d.ny + 1);
+            const int znodes = cath ? d.Lz : d.nz + 1;
+            launch_begin(ctx, K_GREEN_F);
+            if (!a.pot)
+                hipLaunchKernelGGL(k_green_f3<sizeof(T) == 4>,
+                                   dim3((unsigned)div_up(plane, 256), div_up(znodes, kF3Planes), cath ? 2 : 1),
+                                   dim3(256), 0, st, ws.F, a, (const SBunch *)nullptr, 0);
+            else
+                hipLaunchKernelGGL(k_green_f<sizeof(T) == 4>,
+                                   dim3((unsigned)div_up(plane, 256), znodes, ncomp), dim3(256), 0, st,
+                                   ws.F, a, (const SBunch *)nullptr, 0);
+            launch_end(ctx, K_GREEN_F);
+        }
+        launch_begin(ctx, K_GREEN_X);
+        if (engine_of(m, d.Lx, false) == kGeneric ||
+            !green_pass_fast<T>(1, d.Lx, ncomp, d, cath, st, ws, a, twx)) {
+            with_fft_elems<T>(d.Lx, [&](auto e, auto t) {
+                constexpr int E = decltype(e)::value, NT = decltype(t)::value;
+                const int nb = pick_nb(d.Lx, E * NT, 16);
+                const int zc = cath ? d.Lz - 1 : d.nz;
+                const int np = zc * ((d.ny + 1) / 2);
+                const size_t sh = sizeof(cpx<T>) * (d.Lx + (size_t)nb * d.Lx);
+                hipLaunchKernelGGL((k_green_1<T, E, NT>), dim3(div_up(np, nb), ncomp), dim3(NT), sh,
+                                   st, (const double *)ws.F, R, twx, ws.plan[0], a, nb);
+            });
+        }
+        launch_end(ctx, K_GREEN_X);
     }
-    launch_end(ctx, K_GREEN_X);
     const int kp = (d.Kx + 1) / 2;
     launch_begin(ctx, K_GREEN_Y);
     if (engine_of(m, d.Ly, false) == kGeneric ||
@@ -1258,7 +1462,9 @@ void build_green_grouped(const Mesh *m0, int nb, const SBunch *tab, double gamma
     const cpx<T> *tw[3] = {static_cast<const cpx<T> *>(ws.twT[0]),
                            static_cast<const cpx<T> *>(ws.twT[1]),
                            static_cast<const cpx<T> *>(ws.twT[2])};
-    {
+    const bool fused = green_fused(m0, d, sizeof(T), cath) &&
+                       green_fx<T>(d.Lx, d, cath, st, nullptr, a, tw[0], tab, nb);
+    if (!fused) {
         const int per = div_up((d.nx + 1) * (d.ny + 1), 256);
         const int znodes = cath ? d.Lz : d.nz + 1;
         hipLaunchKernelGGL(k_green_f3<sizeof(T) == 4>,
@@ -1267,7 +1473,7 @@ void build_green_grouped(const Mesh *m0, int nb, const SBunch *tab, double gamma
     }
     const int zc = cath ? d.Lz - 1 : d.nz;
     const int kp = (d.Kx + 1) / 2;
-    for (int pass = 1; pass <= 3; ++pass) {
+    for (int pass = fused ? 2 : 1; pass <= 3; ++pass) {
         const int L = pass == 1 ? d.Lx : (pass == 2 ? d.Ly : d.Lz);
         auto go = [&](auto lc) {
             constexpr int LL = decltype(lc)::value;

@@ -43,8 +43,6 @@ namespace sc {
 
 namespace {
 
-constexpr int64_t kInlineGreenBytes = 640 << 10;  // largest Green spectrum built inline (green_overlap)
-
 // ---------------------------------------------------------------------------
 // x pass of the real input: rows (y, z) of component blockIdx.y, zero-padded
 // to 2nx, kx in [0, nx] to that component's spectrum.
@@ -353,18 +351,6 @@ int upload_twiddles(Ctx *ctx, int n, void **dst)
     return SC_OK;
 }
 
-// Whether the Green build overlaps the deposit on the side stream.  The events
-// that fork and join the stream cost the host 24 us a solve, more than a small
-// build takes on the GPU: those run on the caller's stream.  Measured, step of
-// 10k particles on 16^3 on the side stream / inline 100 / 60 us, 100k on 32^3
-// 98 / 76, 200k on 48^3 Float32 115 / 104 but Float64 116 / 124, 1M on 64^3
-// 124 / 136; with the cathode 50k on 32^3 101 / 75, on 48^3 Float64 109 / 113.
-bool green_overlap(const Dims &d, size_t size, int cath)
-{
-    const int64_t nodes = (int64_t)(d.nx + 1) * (d.ny + 1) * (d.nz + 1);
-    return nodes * (int64_t)size * (cath ? 2 : 1) > kInlineGreenBytes;
-}
-
 template <typename T>
 int run_solve(Mesh *m, const double lo[3], const double hi[3], const double dl[3], double gamma,
               const SolveIO &io)
@@ -402,7 +388,7 @@ int run_solve(Mesh *m, const double lo[3], const double hi[3], const double dl[3
     const bool cap = stream_capturing(st, &cid);
     bool overlap = false;
     if (!reuse) {
-        overlap = !ctx->in_batch && green_overlap(d, sizeof(T), cath) &&
+        overlap = !ctx->in_batch && !green_small(d, sizeof(T), cath) &&
                   (cap ? ctx->side && ws.green_done && ws.deposit_start : ensure_side_stream(m) == SC_OK);
         if (overlap) {
             // the build forks where this step's deposit started (recorded by

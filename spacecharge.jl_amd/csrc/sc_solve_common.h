@@ -21,6 +21,18 @@ inline bool smooth7(int L)
     return L == 1;
 }
 
+// true when the register engines transform length L
+inline bool reg_length(int L)
+{
+    switch (L) {
+#define X(LL) case LL:
+        SC_MIX_LENGTHS(X)
+#undef X
+        return true;
+    default: return false;
+    }
+}
+
 // Transform half-length of an axis of n nodes: the smallest t >= n whose 2t
 // the register engines transform (sc_fft_mix.h), on axes beyond those lengths
 // (n > 256) the smallest whose 2t has no prime factor above 7.  The reference
@@ -37,17 +49,6 @@ inline bool smooth7(int L)
 // points, 2994 -> 1531 us in Float32 and 4748 -> 2584 us in Float64; 101^3,
 // 210 -> 256, 386 -> 162 and 549 -> 269 us; 161^3 Float64 with the cathode,
 // 324 -> 384, 3377 -> 2861 us).
-inline bool reg_length(int L)
-{
-    switch (L) {
-#define X(LL) case LL:
-        SC_MIX_LENGTHS(X)
-#undef X
-        return true;
-    default: return false;
-    }
-}
-
 inline int transform_half(int n, bool smooth)
 {
     int t = n;
@@ -193,6 +194,19 @@ __device__ __forceinline__ void zconv_pencils(int task, int nbx, int Ly, int &bx
     const int u = task / nbx;
     const int kyp = (u + 1) >> 1;
     ky = u == 0 ? 0 : ((u & 1) ? kyp : Ly - kyp);
+}
+
+// Small Green builds run on the caller's stream, the others overlap the deposit
+// on the side stream.  The events that fork and join the stream cost the host
+// 24 us a solve, more than a small build takes on the GPU.  Measured, step of
+// 10k particles on 16^3 on the side stream / inline 100 / 60 us, 100k on 32^3
+// 98 / 76, 200k on 48^3 Float32 115 / 104 but Float64 116 / 124, 1M on 64^3
+// 124 / 136; with the cathode 50k on 32^3 101 / 75, on 48^3 Float64 109 / 113.
+constexpr int64_t kSmallGreenBytes = 640 << 10;
+inline bool green_small(const Dims &d, size_t size, int cath)
+{
+    const int64_t nodes = (int64_t)(d.nx + 1) * (d.ny + 1) * (d.nz + 1);
+    return nodes * (int64_t)size * (cath ? 2 : 1) <= kSmallGreenBytes;
 }
 
 // Builds the transformed Green functions for green_mode `mode` into ws.Gf

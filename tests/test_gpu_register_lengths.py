@@ -98,3 +98,30 @@ def test_float64_particles_keep_a_float32_mesh_on_the_generic_engine(grid):
         sc.solve(m)
         out.append(torch.stack(sc.interpolate_field(m, x, y, z)))
     assert out[0].dtype == torch.float64 and torch.equal(out[0], out[1])
+
+
+# Green builds of the fused kernel: several z planes per workgroup and a ragged
+# last group, rows that end inside a workgroup's strip, and (last) an F lattice
+# beyond the 256 MB last-level cache.
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,tol", [(torch.float64, 1e-12), (torch.float32, 1e-5)])
+@pytest.mark.parametrize("grid", [(3, 2, 2), (9, 30, 250), (12, 7, 199), (100, 9, 31), (16, 16, 300),
+                                  (64, 512, 350)])
+def test_fused_green_build_matches_separate_passes(grid, T, tol):
+    import spacecharge as sc
+    dev = torch.device("cuda:0")
+    rho = torch.rand(grid, generator=torch.Generator(device=dev).manual_seed(9), device=dev, dtype=T)
+    worst = 0.0
+    for cath in (False, True):
+        out = []
+        for generic in (False, True):
+            m = sc.Mesh3D(grid, (-1e-3, -1e-3, 1e-4), (1e-3, 1.2e-3, 2e-3), T=T, gamma=2.0)
+            if generic:
+                m.force_generic_transforms()
+            m.rho.copy_(rho)
+            sc.solve(m, at_cathode=cath)
+            out.append(m.efield.cpu().numpy())
+            del m
+        worst = max(worst, max(rel_l2(out[0][..., c], out[1][..., c]) for c in range(3)))
+    print(f"fused Green build {grid} {T}: {worst:.2e}")
+    assert worst <= tol
