@@ -97,7 +97,7 @@ struct V4<double> {
     using type = double4;
 };
 
-// Large Float64 meshes (P = 2) store node pairs: entry i holds nodes i and
+// Float64 meshes (P = 2) store node pairs: entry i holds nodes i and
 // i + 1 (the next node along x; zero past the row's end, which no cell
 // reads), 64 bytes, so that a cell's two x neighbours never straddle a
 // 128-byte line.  Measured on 4M particles, 128^3: the gather 307 -> 245 us,
@@ -110,8 +110,13 @@ struct V4<double> {
 // gather 215 -> 194 us, the copy 45 -> 48 us.  Packed, pairs also pay on
 // smaller Float64 meshes (1M particles, 64^3: gather 46 -> 36 us, step
 // 0.167 -> 0.161 ms; the 2M cathode bunch on 64x64x128: 103 -> 92 us), so
-// every Float64 mesh takes them.  With P = 2 a lane writes one 16-byte
-// quarter of an entry, so the stores are contiguous.
+// Float64 meshes of up to kPairNodes nodes take them.  Beyond, the 64 bytes a
+// node outgrow the 256 MB last-level cache and one node per entry wins again
+// (copy and gather, pairs / single: 4M particles on 160^3 313 / 280 us, 8M on
+// 256^3 1243 / 944; 2M on 128^3 130 / 153).  With P = 2 a lane writes one
+// 16-byte quarter of an entry, so the stores are contiguous.
+constexpr int64_t kPairNodes = 3200000;  // 205 MB of 64-byte entries
+
 template <typename MT>
 __device__ __forceinline__ void interleave_body(int64_t i, const MT *__restrict__ ef,
                                                 typename V4<MT>::type *__restrict__ efi, int64_t M,
@@ -252,6 +257,75 @@ k_interp(const typename V4<MT>::type *__restrict__ efi, const PT *__restrict__ p
 {
     interp_body<PT, MT, PP>((int64_t)blockIdx.x * blockDim.x + threadIdx.x, efi, px, py, pz, n, nx,
                             ny, nz, lx_, ly_, lz_, dx_, dy_, dz_, geom, Ex, Ey, Ez, P);
+}
+
+// The gather straight from the three component arrays, without the interleaved
+// copy (gather_direct): per component four x-neighbour pairs, each one load of two values.
+// The same values and sums as k_interp, so the same bits.
+template <typename T>
+struct Pair {
+    T lo, hi;
+};
+template <typename T>
+__device__ __forceinline__ Pair<T> load_pair(const T *p)
+{
+    // one load of two values, aligned as one
+    Pair<T> v;
+    __builtin_memcpy(&v, p, sizeof(v));
+    return v;
+}
+
+template <typename PT, typename MT>
+__global__ void __launch_bounds__(256)
+k_interp_soa(const MT *__restrict__ ef, const PT *__restrict__ px, const PT *__restrict__ py,
+             const PT *__restrict__ pz, int64_t n, int nx, int ny, int nz, double lx_, double ly_,
+             double lz_, double dx_, double dy_, double dz_, const double *__restrict__ geom,
+             PT *__restrict__ Ex, PT *__restrict__ Ey, PT *__restrict__ Ez)
+{
+#pragma clang fp contract(off)
+    using C = wider_t<PT, MT>;
+    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= n) return;
+    device_geometry(geom, lx_, ly_, lz_, dx_, dy_, dz_);
+    const C lx = (C)(MT)lx_, ly = (C)(MT)ly_, lz = (C)(MT)lz_;
+    const C ddx = (C)(MT)dx_, ddy = (C)(MT)dy_, ddz = (C)(MT)dz_;
+    const C nxn = ((C)px[p] - lx) / ddx;
+    const C nyn = ((C)py[p] - ly) / ddy;
+    const C nzn = ((C)pz[p] - lz) / ddz;
+    const int ix = cell_index(nxn, nx), iy = cell_index(nyn, ny), iz = cell_index(nzn, nz);
+    const C dx = nxn - (C)ix, dy = nyn - (C)iy, dz = nzn - (C)iz;
+    const C one = (C)1;
+    const C w000 = ((one - dx) * (one - dy)) * (one - dz);
+    const C w100 = (dx * (one - dy)) * (one - dz);
+    const C w010 = ((one - dx) * dy) * (one - dz);
+    const C w110 = (dx * dy) * (one - dz);
+    const C w001 = ((one - dx) * (one - dy)) * dz;
+    const C w101 = (dx * (one - dy)) * dz;
+    const C w011 = ((one - dx) * dy) * dz;
+    const C w111 = (dx * dy) * dz;
+    const int64_t sy = nx, sz = (int64_t)nx * ny, M = sz * nz;
+    const MT *e = ef + (ix + sy * iy + sz * iz);
+    Pair<MT> v[3][4];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        v[c][0] = load_pair(e + c * M);
+        v[c][1] = load_pair(e + c * M + sy);
+        v[c][2] = load_pair(e + c * M + sz);
+        v[c][3] = load_pair(e + c * M + sz + sy);
+    }
+    C out[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+        // the reference's sum order (src/interpolation.jl:56-85)
+        out[c] = ((((((((C)v[c][0].lo * w000 + (C)v[c][0].hi * w100) + (C)v[c][1].lo * w010) +
+                      (C)v[c][1].hi * w110) +
+                     (C)v[c][2].lo * w001) +
+                    (C)v[c][2].hi * w101) +
+                   (C)v[c][3].lo * w011) +
+                  (C)v[c][3].hi * w111);
+    Ex[p] = (PT)out[0];
+    Ey[p] = (PT)out[1];
+    Ez[p] = (PT)out[2];
 }
 
 // ---- vector-Jacobian products of the CIC weights ----
@@ -608,10 +682,10 @@ int ensure_efi(Mesh *m)
 {
     if (!m->efi) {
         const int64_t M = m->n[0] * m->n[1] * m->n[2];
-        // node pairs for Float64 fields (see interleave_body), unless the
-        // mesh asks for a layout
+        // node pairs for Float64 fields of up to kPairNodes nodes (see
+        // interleave_body), unless the mesh asks for a layout
         if (m->efi_layout) m->efi_pair = m->efi_layout;
-        else m->efi_pair = m->dtype == SC_F64 ? 2 : 1;
+        else m->efi_pair = m->dtype == SC_F64 && M <= kPairNodes ? 2 : 1;
         if (hipMalloc(&m->efi, (size_t)M * 4 * m->dtype * m->efi_pair) != hipSuccess)
             return set_err(m->ctx, SC_ERR_NOMEM, "device allocation of the interleaved field failed");
     }
@@ -694,10 +768,56 @@ int launch_interp_into(Mesh *m, void *efi, int P, int pdt, const void *x, const 
     return SC_OK;
 }
 
+namespace {
+
+template <typename PT, typename MT>
+void itp_soa(Mesh *m, const void *x, const void *y, const void *z, int64_t n, const double lo[3],
+             const double dl[3], void *Ex, void *Ey, void *Ez)
+{
+    const LaunchGeo h = launch_geo(m, lo, dl);
+    hipLaunchKernelGGL((k_interp_soa<PT, MT>), dim3((unsigned)blocks_for(n, 256)), dim3(256), 0,
+                       m->ctx->stream, (const MT *)m->efield, (const PT *)x, (const PT *)y,
+                       (const PT *)z, n, (int)m->n[0], (int)m->n[1], (int)m->n[2], h.l[0], h.l[1],
+                       h.l[2], h.d[0], h.d[1], h.d[2], h.dev, (PT *)Ex, (PT *)Ey, (PT *)Ez);
+}
+
+// Whether the interpolation of n particles gathers straight from efield: the
+// interleaved copy costs a launch and a pass over all M nodes, the direct
+// gather two to three times the cache lines per particle, so few particles per
+// node go direct.  Measured, direct / interleaved (us), Float32: 200k on 128^3
+// (0.10 per node) 17 / 21, 500k (0.24) 31 / 28; 50k on 32^3 4.9 / 7.1, 200k on
+// 64^3 14 / 13; 500k on 256^3 (0.03) 81 / 111, 1M (0.06) 155 / 141.  Float64: 1M on
+// 128^3 (0.48) 80 / 87, 2M 148 / 130; 200k on 32^3 12 / 14, 500k 22.5 / 21; 1M on
+// 256^3 (0.06) 199 / 274, 2M (0.12) 389 / 367.  A forced layout keeps its copy.
+bool gather_direct(const Mesh *m, int64_t n)
+{
+    if (m->efi_layout) return false;
+    const int64_t M = m->n[0] * m->n[1] * m->n[2];
+    if (m->dtype == SC_F32) {
+        const int64_t few = M > 6000000 ? M / 20 : M / 6;
+        return n <= (few > 131072 ? few : 131072);
+    }
+    const int64_t few = M > kPairNodes ? M / 8 : M / 2;
+    return n <= (few > 400000 ? few : 400000);
+}
+
+}  // namespace
+
 int launch_interp(Mesh *m, int pdt, const void *x, const void *y, const void *z, int64_t n,
                   const double lo[3], const double dl[3], void *Ex, void *Ey, void *Ez)
 {
     if (n <= 0) return SC_OK;
+    if (gather_direct(m, n)) {
+        launch_begin(m->ctx, K_INTERP);
+        if (pdt == SC_F32 && m->dtype == SC_F32) itp_soa<float, float>(m, x, y, z, n, lo, dl, Ex, Ey, Ez);
+        else if (pdt == SC_F64 && m->dtype == SC_F64)
+            itp_soa<double, double>(m, x, y, z, n, lo, dl, Ex, Ey, Ez);
+        else if (pdt == SC_F64) itp_soa<double, float>(m, x, y, z, n, lo, dl, Ex, Ey, Ez);
+        else itp_soa<float, double>(m, x, y, z, n, lo, dl, Ex, Ey, Ez);
+        launch_end(m->ctx, K_INTERP);
+        SC_HIP(m->ctx, hipGetLastError());
+        return SC_OK;
+    }
     if (int rc = ensure_efi(m)) return rc;
     return launch_interp_into(m, m->efi, m->efi_pair, pdt, x, y, z, n, lo, dl, Ex, Ey, Ez);
 }

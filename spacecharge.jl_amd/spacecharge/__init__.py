@@ -296,8 +296,8 @@ class Mesh3D:
     def set_field_layout(self, layout: int = 0) -> None:
         """Diagnostic: layout of the interpolation's node-interleaved field
         copy: 1 = one entry per node, 2 = node pairs along x (Float64 meshes
-        only; picked by the library for Float64 fields of 64 MiB and more),
-        0 = by size."""
+        only), 0 = picked by the library (node pairs for Float64 meshes of up
+        to 3.2M nodes, and no copy at all for few particles per node)."""
         ctx = _ctx(self.device)
         with _on(self.device):
             rc = _lib.load().sc_mesh_set_field_layout(self._h, int(layout))
