@@ -105,11 +105,11 @@ int sc_mesh_set_green_reuse(sc_mesh *mesh, int enable);
 int sc_mesh_force_generic_transforms(sc_mesh *mesh, int enable);
 /* Diagnostic (no reference counterpart): the layout of the node-interleaved
  * field copy that the interpolation and its adjoint gather from.  layout 1
- * holds one (Ex, Ey, Ez, 0) entry per node; layout 2 holds node pairs (nodes
- * i and i+1 along x per entry; Float64 meshes only), which the library
- * picks by itself for Float64 meshes of up to 3.2 million nodes; 0 (the
- * default) restores that choice, and gathers without a copy where the
- * particles are few per node.
+ * holds one padded (Ex, Ey, Ez, 0) entry per node; layout 2 packs the three
+ * values of a node, so that the node pairs of a cell along x are one run of six
+ * (Float64 meshes only; the library also picks it for Float32 meshes of more
+ * than 8 million nodes); 0 (the default) lets the library choose: packed for
+ * Float64 meshes, and no copy at all where the particles are few per node.
  * Results are the same bits in every layout.  Changing it synchronises the
  * context's stream and frees the current copy. */
 int sc_mesh_set_field_layout(sc_mesh *mesh, int layout);

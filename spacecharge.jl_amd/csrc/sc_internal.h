@@ -234,7 +234,7 @@ struct Mesh {
     Workspace ws;
     DepositBins bins;
     void *efi = nullptr;  // node-interleaved field for the interpolation gather
-    int efi_pair = 1;     // entries per node in efi: 2 = node pairs (Float64 meshes, ensure_efi)
+    int efi_pair = 1;     // layout of efi: 1 = a padded entry per node, 2 = packed (ensure_efi)
     int efi_layout = 0;   // requested efi_pair: 0 = by size (ensure_efi), 1 or 2 = forced
     // device-resident geometry (lo[3], hi[3], delta[3] as doubles holding
     // mesh-type values), written by sc_mesh_auto_bounds on the stream; the
@@ -340,7 +340,7 @@ void free_bins(Mesh *m);
 int launch_interp(Mesh *m, int pdt, const void *x, const void *y, const void *z, int64_t n,
                   const double lo[3], const double dl[3], void *Ex, void *Ey, void *Ez);
 // launch_interp with the node-interleaved field copy in the caller's buffer
-// `efi` (P entries per node, nx*ny*nz*P*4 mesh-type values); allocates nothing.
+// `efi` (layout P, nx*ny*nz*4 mesh-type values at most); allocates nothing.
 int launch_interp_into(Mesh *m, void *efi, int P, int pdt, const void *x, const void *y,
                        const void *z, int64_t n, const double lo[3], const double dl[3], void *Ex,
                        void *Ey, void *Ez);

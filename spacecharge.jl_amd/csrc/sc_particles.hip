@@ -97,80 +97,72 @@ struct V4<double> {
     using type = double4;
 };
 
-// Float64 meshes (P = 2) store node pairs: entry i holds nodes i and
-// i + 1 (the next node along x; zero past the row's end, which no cell
-// reads), 64 bytes, so that a cell's two x neighbours never straddle a
-// 128-byte line.  Measured on 4M particles, 128^3: the gather 307 -> 245 us,
-// the copy 26 -> 47 us, the step 0.834 -> 0.792 ms.  Float32 meshes keep one
-// node per entry (16-byte nodes straddle a line in one pair of eight; on 4M
-// particles, 128^3, pairs took the gather from 99 to 134 us).
-// The six values of a pair are packed (Ex, Ey, Ez of node i, then of node
-// i + 1, then 16 bytes of zeros), so a gather of both nodes is three
-// 16-byte loads (pair_nodes) instead of four: on 4M particles, 128^3, the
-// gather 215 -> 194 us, the copy 45 -> 48 us.  Packed, pairs also pay on
-// smaller Float64 meshes (1M particles, 64^3: gather 46 -> 36 us, step
-// 0.167 -> 0.161 ms; the 2M cathode bunch on 64x64x128: 103 -> 92 us), so
-// Float64 meshes of up to kPairNodes nodes take them.  Beyond, the 64 bytes a
-// node outgrow the 256 MB last-level cache and one node per entry wins again
-// (copy and gather, pairs / single: 4M particles on 160^3 313 / 280 us, 8M on
-// 256^3 1243 / 944; 2M on 128^3 130 / 153).  With P = 2 a lane writes one
-// 16-byte quarter of an entry, so the stores are contiguous.
-constexpr int64_t kPairNodes = 3200000;  // 205 MB of 64-byte entries
+// Two layouts.  P = 1: one padded entry (Ex, Ey, Ez, 0) per node, one aligned
+// vector load each.  P = 2, packed: the three values of a node only, so that a
+// cell's x neighbours are one run of six (three 16-byte loads in Float64) and
+// the copy is a quarter smaller.  The gather is bound by the cache lines that
+// its random rows miss, in the L1 while the copy is small and in the L2 and the
+// last-level cache as it grows.  Measured (copy and gather, us), Float64, P = 1 /
+// node pairs padded to 64 bytes, an earlier layout / P = 2: 4M particles on 128^3
+// - / 231 / 173, the 2M cathode bunch on 64x64x128 - / 99 / 80, 1M on 64^3 53 / 49
+// / 38, 8M on 256^3 944 / 1243 / 750: packed for every Float64 mesh.  Float32, P =
+// 1 / 2: 128^3 104 / 119 (the 24-byte runs straddle 16 bytes), 160^3 78 / 81, 256^3
+// 504 / 437: packed beyond kPackedNodes32 nodes, where the padded copy outgrows
+// the last-level cache.
+constexpr int64_t kPackedNodes32 = 8000000;
 
 template <typename MT>
 __device__ __forceinline__ void interleave_body(int64_t i, const MT *__restrict__ ef,
                                                 typename V4<MT>::type *__restrict__ efi, int64_t M,
-                                                int nx, int P)
+                                                int P)
 {
-    if constexpr (sizeof(MT) == 8) {
-        if (P == 2) {
-            if (i >= 4 * M) return;
-            const int64_t e = i >> 2;
-            const int part = (int)(i & 3);
-            const bool hi = e % nx != nx - 1;  // node e + 1 is in the row
-            // values 2 part and 2 part + 1 of the entry's six: value s is
-            // component s % 3 of node e + s / 3 (no branch per quarter)
-            const int s0 = 2 * part, s1 = s0 + 1;
-            const bool ok0 = s0 < 3 || (s0 < 6 && hi), ok1 = s1 < 3 || (s1 < 6 && hi);
-            const int64_t i0 = ok0 ? (s0 % 3) * M + e + s0 / 3 : 0;
-            const int64_t i1 = ok1 ? (s1 % 3) * M + e + s1 / 3 : 0;
-            const double a = ef[i0], b = ef[i1];
-            // streamed past the L2: a pair copy (64 bytes per node) outgrows
-            // it anyway, and the gather then finds it in the last-level cache
-            // (4M particles, 128^3: the copy 47.5 -> 34.1 us, the gather
-            // 194.4 -> 196.8 us).  The padding quarter is written too: left
-            // out, the partial lines made the copy slower (55 us).
-            double *dst = reinterpret_cast<double *>(efi) + 2 * i;
-            __builtin_nontemporal_store(ok0 ? a : 0.0, dst);
-            __builtin_nontemporal_store(ok1 ? b : 0.0, dst + 1);
-            return;
-        }
-    }
     if (i >= M) return;
+    const MT a = ef[i], b = ef[M + i], c = ef[2 * M + i];
+    if (P == 2) {
+        MT *o = reinterpret_cast<MT *>(efi) + 3 * i;
+        o[0] = a;
+        o[1] = b;
+        o[2] = c;
+        return;
+    }
     typename V4<MT>::type v;
-    v.x = ef[i];
-    v.y = ef[M + i];
-    v.z = ef[2 * M + i];
+    v.x = a;
+    v.y = b;
+    v.z = c;
     v.w = (MT)0;
     efi[i] = v;
 }
 
 template <typename MT>
 __global__ void __launch_bounds__(256)
-k_interleave(const MT *__restrict__ ef, typename V4<MT>::type *__restrict__ efi, int64_t M, int nx,
-             int P)
+k_interleave(const MT *__restrict__ ef, typename V4<MT>::type *__restrict__ efi, int64_t M, int P)
 {
-    interleave_body<MT>((int64_t)blockIdx.x * blockDim.x + threadIdx.x, ef, efi, M, nx, P);
+    interleave_body<MT>((int64_t)blockIdx.x * blockDim.x + threadIdx.x, ef, efi, M, P);
 }
 
-// Nodes i and i + 1 of a packed node-pair entry (Float64, P = 2): the
-// first 32 bytes and the next 16, as two one-node entries.
-__device__ __forceinline__ void pair_nodes(const double4 *__restrict__ ent, double4 &lo, double4 &hi)
+// The eight nodes of the cell with lower corner `node`, in the order x, y, z
+// fastest to slowest, from either layout.
+template <typename MT, int P>
+__device__ __forceinline__ void cell_nodes(const typename V4<MT>::type *__restrict__ efi, int64_t node,
+                                           int64_t nx, int64_t nxy, typename V4<MT>::type *nd)
 {
-    const double4 a = ent[0];
-    const double2 b = *reinterpret_cast<const double2 *>(ent + 1);
-    lo = make_double4(a.x, a.y, a.z, 0.0);
-    hi = make_double4(a.w, b.x, b.y, 0.0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int64_t i = node + (r & 1 ? nx : 0) + (r & 2 ? nxy : 0);
+        if constexpr (P == 2) {
+            MT v[6];  // one run, aligned as a single value
+            __builtin_memcpy(v, reinterpret_cast<const MT *>(efi) + 3 * i, sizeof(v));
+            nd[2 * r] = {v[0], v[1], v[2], (MT)0};
+            nd[2 * r + 1] = {v[3], v[4], v[5], (MT)0};
+        } else {
+            nd[2 * r] = efi[i];
+            nd[2 * r + 1] = efi[i + 1];
+        }
+        // row by row, arithmetic free to move: left to itself the compiler put the
+        // last loads of the rows at the end, where the L1 no longer held their lines
+        // (4M particles, 128^3 Float64: copy and gather 207 us, so 173)
+        __builtin_amdgcn_sched_barrier(0x7);
+    }
 }
 
 // PP: the entry layout when known at compile time (1 or 2), else 0 and P
@@ -213,27 +205,12 @@ __device__ __forceinline__ void interp_body(
     const C w101 = (dx * (one - dy)) * dz;
     const C w011 = ((one - dx) * dy) * dz;
     const C w111 = (dx * dy) * dz;
-    const int64_t sy = (int64_t)P * nx, sz = (int64_t)P * nx * ny;
-    const typename V4<MT>::type *e = efi + P * (ix + (int64_t)nx * iy + (int64_t)nx * ny * iz);
-    typename V4<MT>::type n000, n100, n010, n110, n001, n101, n011, n111;
-    if constexpr (sizeof(MT) == 8) {
-        if (PP == 2) {
-            pair_nodes(e, n000, n100);
-            pair_nodes(e + sy, n010, n110);
-            pair_nodes(e + sz, n001, n101);
-            pair_nodes(e + sz + sy, n011, n111);
-        } else {
-            n000 = e[0], n100 = e[1], n010 = e[sy], n110 = e[sy + 1];
-            n001 = e[sz], n101 = e[sz + 1], n011 = e[sz + sy], n111 = e[sz + sy + 1];
-        }
-    } else {
-        n000 = e[0], n100 = e[1], n010 = e[sy], n110 = e[sy + 1];
-        n001 = e[sz], n101 = e[sz + 1], n011 = e[sz + sy], n111 = e[sz + sy + 1];
-    }
+    typename V4<MT>::type nd[8];
+    cell_nodes<MT, PP>(efi, ix + (int64_t)nx * iy + (int64_t)nx * ny * iz, nx, (int64_t)nx * ny, nd);
     // the reference's sum order, per component (src/interpolation.jl:56-85)
 #define SC_ITP(f)                                              \
-    ((((((((C)n000.f * w000 + (C)n100.f * w100) + (C)n010.f * w010) + (C)n110.f * w110) + \
-         (C)n001.f * w001) + (C)n101.f * w101) + (C)n011.f * w011) + (C)n111.f * w111)
+    ((((((((C)nd[0].f * w000 + (C)nd[1].f * w100) + (C)nd[2].f * w010) + (C)nd[3].f * w110) + \
+         (C)nd[4].f * w001) + (C)nd[5].f * w101) + (C)nd[6].f * w011) + (C)nd[7].f * w111)
     Ex[p] = (PT)SC_ITP(x);
     Ey[p] = (PT)SC_ITP(y);
     Ez[p] = (PT)SC_ITP(z);
@@ -276,15 +253,14 @@ __device__ __forceinline__ Pair<T> load_pair(const T *p)
 }
 
 template <typename PT, typename MT>
-__global__ void __launch_bounds__(256)
-k_interp_soa(const MT *__restrict__ ef, const PT *__restrict__ px, const PT *__restrict__ py,
-             const PT *__restrict__ pz, int64_t n, int nx, int ny, int nz, double lx_, double ly_,
-             double lz_, double dx_, double dy_, double dz_, const double *__restrict__ geom,
-             PT *__restrict__ Ex, PT *__restrict__ Ey, PT *__restrict__ Ez)
+__device__ __forceinline__ void interp_soa_body(
+    int64_t p, const MT *__restrict__ ef, const PT *__restrict__ px, const PT *__restrict__ py,
+    const PT *__restrict__ pz, int64_t n, int nx, int ny, int nz, double lx_, double ly_, double lz_,
+    double dx_, double dy_, double dz_, const double *__restrict__ geom, PT *__restrict__ Ex,
+    PT *__restrict__ Ey, PT *__restrict__ Ez)
 {
 #pragma clang fp contract(off)
     using C = wider_t<PT, MT>;
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= n) return;
     device_geometry(geom, lx_, ly_, lz_, dx_, dy_, dz_);
     const C lx = (C)(MT)lx_, ly = (C)(MT)ly_, lz = (C)(MT)lz_;
@@ -326,6 +302,17 @@ k_interp_soa(const MT *__restrict__ ef, const PT *__restrict__ px, const PT *__r
     Ex[p] = (PT)out[0];
     Ey[p] = (PT)out[1];
     Ez[p] = (PT)out[2];
+}
+
+template <typename PT, typename MT>
+__global__ void __launch_bounds__(256)
+k_interp_soa(const MT *__restrict__ ef, const PT *__restrict__ px, const PT *__restrict__ py,
+             const PT *__restrict__ pz, int64_t n, int nx, int ny, int nz, double lx_, double ly_,
+             double lz_, double dx_, double dy_, double dz_, const double *__restrict__ geom,
+             PT *__restrict__ Ex, PT *__restrict__ Ey, PT *__restrict__ Ez)
+{
+    interp_soa_body<PT, MT>((int64_t)blockIdx.x * blockDim.x + threadIdx.x, ef, px, py, pz, n, nx, ny,
+                            nz, lx_, ly_, lz_, dx_, dy_, dz_, geom, Ex, Ey, Ez);
 }
 
 // ---- vector-Jacobian products of the CIC weights ----
@@ -422,29 +409,8 @@ k_interp_vjp(const typename V4<MT>::type *__restrict__ efi, const PT *__restrict
     const C nzn = ((C)pz[p] - (C)(MT)lz_) / ddz;
     const int ix = cell_index(nxn, nx), iy = cell_index(nyn, ny), iz = cell_index(nzn, nz);
     const C dx = nxn - (C)ix, dy = nyn - (C)iy, dz = nzn - (C)iz;
-    const int64_t sy = (int64_t)P * nx, sz = (int64_t)P * nx * ny;
-    const typename V4<MT>::type *e = efi + P * (ix + (int64_t)nx * iy + (int64_t)nx * ny * iz);
     typename V4<MT>::type nd[8];
-    bool packed = false;
-    if constexpr (sizeof(MT) == 8) {
-        if (PP == 2) {
-            pair_nodes(e, nd[0], nd[1]);
-            pair_nodes(e + sy, nd[2], nd[3]);
-            pair_nodes(e + sz, nd[4], nd[5]);
-            pair_nodes(e + sz + sy, nd[6], nd[7]);
-            packed = true;
-        }
-    }
-    if (!packed) {
-        nd[0] = e[0];
-        nd[1] = e[1];
-        nd[2] = e[sy];
-        nd[3] = e[sy + 1];
-        nd[4] = e[sz];
-        nd[5] = e[sz + 1];
-        nd[6] = e[sz + sy];
-        nd[7] = e[sz + sy + 1];
-    }
+    cell_nodes<MT, PP>(efi, ix + (int64_t)nx * iy + (int64_t)nx * ny * iz, nx, (int64_t)nx * ny, nd);
     C f[8], val, Gx, Gy, Gz;
     C sx = (C)0, sy_ = (C)0, sz_ = (C)0;
 #pragma unroll
@@ -622,15 +588,14 @@ void dep(Mesh *m, const void *x, const void *y, const void *z, const void *q, in
                        h.d[0], h.d[1], h.d[2], h.dev);
 }
 
-// The node-interleaved copy of m->efield in `efi` (P entries per node).
+// The node-interleaved copy of m->efield in `efi` (layout P).
 template <typename MT>
 void interleave(Mesh *m, void *efi, int P)
 {
     const int64_t M = m->n[0] * m->n[1] * m->n[2];
-    hipLaunchKernelGGL((k_interleave<MT>), dim3((unsigned)blocks_for(P == 2 ? 4 * M : M, 256)),
-                       dim3(256), 0,
+    hipLaunchKernelGGL((k_interleave<MT>), dim3((unsigned)blocks_for(M, 256)), dim3(256), 0,
                        m->ctx->stream, (const MT *)m->efield,
-                       static_cast<typename V4<MT>::type *>(efi), M, (int)m->n[0], P);
+                       static_cast<typename V4<MT>::type *>(efi), M, P);
 }
 
 template <typename PT, typename MT>
@@ -678,15 +643,36 @@ void itp_vjp(Mesh *m, const void *x, const void *y, const void *z, int64_t n, co
                        accumulate, m->efi_pair);
 }
 
+// Whether the interpolation of n particles gathers straight from efield: the
+// interleaved copy costs a launch and a pass over all M nodes, the direct
+// gather two to three times the cache lines per particle, so few particles per
+// node go direct; the larger the field, the sooner its lines miss the caches.
+// Measured, direct / interleaved (us), Float32: 200k on 128^3 (0.10 per node) 17 /
+// 21, 500k (0.24) 31 / 28; 50k on 32^3 4.9 / 7.1, 200k on 64^3 14 / 13; 500k on 256^3
+// (0.03) 80 / 100, 1M (0.06) 155 / 125.  Float64: 500k on 128^3 (0.24) 44 / 45, 1M 81 /
+// 66; 200k on 32^3 12 / 12, 500k 22.5 / 18; on 160^3 500k (0.12) 56 / 62, 1M 100 / 86;
+// on 256^3 1M (0.06) 197 / 230, 2M 381 / 304.  A forced layout keeps its copy.
+bool gather_direct(const Mesh *m, int64_t n)
+{
+    if (m->efi_layout) return false;
+    const int64_t M = m->n[0] * m->n[1] * m->n[2];
+    if (m->dtype == SC_F32) {
+        const int64_t few = M > 6000000 ? M / 20 : M / 6;
+        return n <= (few > 131072 ? few : 131072);
+    }
+    const int64_t few = M > 6000000 ? M / 12 : M > 3000000 ? M / 6 : M / 3;
+    return n <= (few > 200000 ? few : 200000);
+}
+
 int ensure_efi(Mesh *m)
 {
     if (!m->efi) {
         const int64_t M = m->n[0] * m->n[1] * m->n[2];
-        // node pairs for Float64 fields of up to kPairNodes nodes (see
+        // packed for Float64 fields and large Float32 ones (see
         // interleave_body), unless the mesh asks for a layout
         if (m->efi_layout) m->efi_pair = m->efi_layout;
-        else m->efi_pair = m->dtype == SC_F64 && M <= kPairNodes ? 2 : 1;
-        if (hipMalloc(&m->efi, (size_t)M * 4 * m->dtype * m->efi_pair) != hipSuccess)
+        else m->efi_pair = m->dtype == SC_F64 || M > kPackedNodes32 ? 2 : 1;
+        if (hipMalloc(&m->efi, (size_t)M * (m->efi_pair == 2 ? 3 : 4) * m->dtype) != hipSuccess)
             return set_err(m->ctx, SC_ERR_NOMEM, "device allocation of the interleaved field failed");
     }
     return SC_OK;
@@ -779,26 +765,6 @@ void itp_soa(Mesh *m, const void *x, const void *y, const void *z, int64_t n, co
                        m->ctx->stream, (const MT *)m->efield, (const PT *)x, (const PT *)y,
                        (const PT *)z, n, (int)m->n[0], (int)m->n[1], (int)m->n[2], h.l[0], h.l[1],
                        h.l[2], h.d[0], h.d[1], h.d[2], h.dev, (PT *)Ex, (PT *)Ey, (PT *)Ez);
-}
-
-// Whether the interpolation of n particles gathers straight from efield: the
-// interleaved copy costs a launch and a pass over all M nodes, the direct
-// gather two to three times the cache lines per particle, so few particles per
-// node go direct.  Measured, direct / interleaved (us), Float32: 200k on 128^3
-// (0.10 per node) 17 / 21, 500k (0.24) 31 / 28; 50k on 32^3 4.9 / 7.1, 200k on
-// 64^3 14 / 13; 500k on 256^3 (0.03) 81 / 111, 1M (0.06) 155 / 141.  Float64: 1M on
-// 128^3 (0.48) 80 / 87, 2M 148 / 130; 200k on 32^3 12 / 14, 500k 22.5 / 21; 1M on
-// 256^3 (0.06) 199 / 274, 2M (0.12) 389 / 367.  A forced layout keeps its copy.
-bool gather_direct(const Mesh *m, int64_t n)
-{
-    if (m->efi_layout) return false;
-    const int64_t M = m->n[0] * m->n[1] * m->n[2];
-    if (m->dtype == SC_F32) {
-        const int64_t few = M > 6000000 ? M / 20 : M / 6;
-        return n <= (few > 131072 ? few : 131072);
-    }
-    const int64_t few = M > kPairNodes ? M / 8 : M / 2;
-    return n <= (few > 400000 ? few : 400000);
 }
 
 }  // namespace
@@ -976,7 +942,7 @@ struct IBunch {
     void *Ex, *Ey, *Ez;
     int64_t n, M;
     double l[3], d[3];
-    int nx, ny, nz, P;  // P: entries per node of efi
+    int nx, ny, nz, P;  // P: layout of efi, 0: gather from ef
 };
 
 struct ITable {
@@ -1025,7 +991,7 @@ __global__ void __launch_bounds__(256) k_interleave_g(const ITable *__restrict__
     const IBunch &d = T->b[b];
     const int64_t lb = blockIdx.x - T->start[kIInterleave][b];
     interleave_body<MT>(lb * blockDim.x + threadIdx.x, static_cast<const MT *>(d.ef),
-                        static_cast<typename V4<MT>::type *>(d.efi), d.M, d.nx, d.P);
+                        static_cast<typename V4<MT>::type *>(d.efi), d.M, d.P);
 }
 
 template <typename PT, typename MT>
@@ -1036,6 +1002,13 @@ k_interp_g(const ITable *__restrict__ T)
     const int b = igroup_of(T->start[kIGather], T->nb, blockIdx.x);
     const IBunch &d = T->b[b];
     const int64_t lb = blockIdx.x - T->start[kIGather][b];
+    if (d.P == 0) {  // straight from efield (gather_direct)
+        interp_soa_body<PT, MT>(lb * blockDim.x + threadIdx.x, static_cast<const MT *>(d.ef),
+                                (const PT *)d.x, (const PT *)d.y, (const PT *)d.z, d.n, d.nx, d.ny,
+                                d.nz, d.l[0], d.l[1], d.l[2], d.d[0], d.d[1], d.d[2], nullptr,
+                                (PT *)d.Ex, (PT *)d.Ey, (PT *)d.Ez);
+        return;
+    }
     interp_body<PT, MT>(lb * blockDim.x + threadIdx.x,
                         static_cast<const typename V4<MT>::type *>(d.efi), (const PT *)d.x,
                         (const PT *)d.y, (const PT *)d.z, d.n, d.nx, d.ny, d.nz, d.l[0], d.l[1],
@@ -1046,10 +1019,12 @@ k_interp_g(const ITable *__restrict__ T)
 template <typename PT, typename MT>
 void launch_igroups(Ctx *ctx, ITable *T, const unsigned *total)
 {
-    launch_begin(ctx, K_INTERLEAVE);
-    hipLaunchKernelGGL(k_interleave_g<MT>, dim3(total[kIInterleave]), dim3(256), 0, ctx->stream,
-                       (const ITable *)T);
-    launch_end(ctx, K_INTERLEAVE);
+    if (total[kIInterleave]) {  // some bunch gathers from a copy
+        launch_begin(ctx, K_INTERLEAVE);
+        hipLaunchKernelGGL(k_interleave_g<MT>, dim3(total[kIInterleave]), dim3(256), 0, ctx->stream,
+                           (const ITable *)T);
+        launch_end(ctx, K_INTERLEAVE);
+    }
     launch_begin(ctx, K_INTERP);
     hipLaunchKernelGGL((k_interp_g<PT, MT>), dim3(total[kIGather]), dim3(256), 0, ctx->stream,
                        (const ITable *)T);
@@ -1077,7 +1052,8 @@ int launch_interp_grouped(Ctx *ctx, Mesh *const *ms, int nb, int pdt, const void
     }
     if (int rc = ensure_group_table(ctx, group_table_bytes())) return rc;
     for (int b = 0; b < nb; ++b)
-        if (int rc = ensure_efi(ms[b])) return rc;
+        if (!gather_direct(ms[b], n[b]))
+            if (int rc = ensure_efi(ms[b])) return rc;
     ITable *T = static_cast<ITable *>(ctx->gtable);
     unsigned total[kIPhases] = {};
     IStore s;
@@ -1107,8 +1083,8 @@ int launch_interp_grouped(Ctx *ctx, Mesh *const *ms, int nb, int pdt, const void
             d.nx = (int)m->n[0];
             d.ny = (int)m->n[1];
             d.nz = (int)m->n[2];
-            d.P = m->efi_pair;
-            const unsigned blocks[kIPhases] = {(unsigned)blocks_for(d.P == 2 ? 4 * d.M : d.M, 256),
+            d.P = gather_direct(m, n[b]) ? 0 : m->efi_pair;
+            const unsigned blocks[kIPhases] = {d.P == 0 ? 0u : (unsigned)blocks_for(d.M, 256),
                                                (unsigned)blocks_for(d.n, 256)};
             for (int ph = 0; ph < kIPhases; ++ph) {
                 s.start[ph][k] = total[ph];

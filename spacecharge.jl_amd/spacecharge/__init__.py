@@ -295,9 +295,10 @@ class Mesh3D:
 
     def set_field_layout(self, layout: int = 0) -> None:
         """Diagnostic: layout of the interpolation's node-interleaved field
-        copy: 1 = one entry per node, 2 = node pairs along x (Float64 meshes
-        only), 0 = picked by the library (node pairs for Float64 meshes of up
-        to 3.2M nodes, and no copy at all for few particles per node)."""
+        copy: 1 = one padded entry per node, 2 = packed, so that the node pairs
+        along x are one run (Float64 meshes only), 0 = picked by the library
+        (packed for Float64 meshes, and no copy at all for few particles per
+        node)."""
         ctx = _ctx(self.device)
         with _on(self.device):
             rc = _lib.load().sc_mesh_set_field_layout(self._h, int(layout))
