@@ -179,26 +179,18 @@ struct Workspace {
     void *twT[3] = {nullptr, nullptr, nullptr};
     FftPlan plan[3];
     // ordering of the Green build on the side stream: green_done after the
-    // build (the z convolution waits for it), gf_free after the z
-    // convolution (the next eager build waits for it; recorded by eager
-    // calls only)
-    hipEvent_t green_done = nullptr, gf_free = nullptr;
-    bool gf_free_recorded = false;
+    // build (the z convolution waits for it)
+    hipEvent_t green_done = nullptr;
     // recorded where each deposit into this mesh starts (mark_deposit_start):
     // the next build forks from it, so that it overlaps the deposit kernels
     // (latency bound) rather than the previous step's interpolation.
-    // fork_ready: recorded by an eager deposit that no build has forked from
-    // yet; start_recorded: an eager record exists (an older one is still a
-    // safe fork point for an eager build, which also waits for gf_free after
-    // the last eager z convolution, as long as no capture has used this
-    // mesh: a graph's z convolutions record no gf_free); captured: a stream
-    // capture has used this mesh's events; fork_capture: the id of the
-    // capture whose deposit recorded the event (0: none).  A build with no
-    // usable record forks from the end of the stream.
+    // fork_ready: recorded by an eager deposit, and no solve of this mesh has
+    // been launched since (its z convolution reads the spectra that the build
+    // writes); fork_capture: the id of the capture whose deposit recorded the
+    // event, likewise (0: none).  A build with no usable record forks from the
+    // end of the stream.
     hipEvent_t deposit_start = nullptr;
     bool fork_ready = false;
-    bool start_recorded = false;
-    bool captured = false;
     unsigned long long fork_capture = 0;
     // cached Green key for the opt-in reuse
     bool g_valid = false;

@@ -392,24 +392,14 @@ int run_solve(Mesh *m, const double lo[3], const double hi[3], const double dl[3
                   (cap ? ctx->side && ws.green_done && ws.deposit_start : ensure_side_stream(m) == SC_OK);
         if (overlap) {
             // the build forks where this step's deposit started (recorded by
-            // a deposit of this capture, or by an eager deposit; an older
-            // eager record only if no capture has used this mesh), else at
-            // the current end of `st`, which may still read this mesh's
-            // Green spectra
-            const bool from_deposit =
-                cap ? ws.fork_capture == cid : (ws.fork_ready || (ws.start_recorded && !ws.captured));
-            if (!from_deposit) {
-                SC_HIP(ctx, hipEventRecord(ws.deposit_start, st));
-                if (!cap) ws.start_recorded = true;
-            }
-            if (cap) ws.captured = true;
-            ws.fork_ready = false;
-            ws.fork_capture = 0;
-            // an eager build also waits for the last eager z convolution,
-            // which may have run on another stream (a graph is ordered by its
-            // launch stream instead)
-            if (!cap && ws.gf_free_recorded)
-                SC_HIP(ctx, hipStreamWaitEvent(ctx->side, ws.gf_free, 0));
+            // a deposit of this capture, or by an eager deposit, and no solve
+            // launched since), else at the current end of `st`.  Both lie after
+            // the last z convolution that reads this mesh's Green spectra: an
+            // event of its own after each of those, for builds that fork
+            // further back, cost 5.5 us of idle device and 3 us of host time
+            // per solve
+            const bool from_deposit = cap ? ws.fork_capture == cid : ws.fork_ready;
+            if (!from_deposit) SC_HIP(ctx, hipEventRecord(ws.deposit_start, st));
             SC_HIP(ctx, hipStreamWaitEvent(ctx->side, ws.deposit_start, 0));
             ctx->stream = ctx->side;  // the build launches (and times) on ctx->stream
             const int rc = build_green<T>(m, dl, gamma, offz, gmode);
@@ -485,10 +475,9 @@ int run_solve(Mesh *m, const double lo[3], const double hi[3], const double dl[3
             launch_end(ctx, K_ZCONV);
         });
     }
-    if (ws.green_done && !cap) {  // the side stream exists: the next build waits for this point
-        SC_HIP(ctx, hipEventRecord(ws.gf_free, st));
-        ws.gf_free_recorded = true;
-    }
+    // a later build without a new deposit forks after this point
+    ws.fork_ready = false;
+    ws.fork_capture = 0;
     // ---- backward y, x ----
     if (!fast(3)) {
         with_fft_elems<T>(d.Ly, [&](auto e, auto t) {
@@ -572,8 +561,6 @@ int mark_deposit_start(Mesh *m)
     SC_HIP(m->ctx, hipEventRecord(ws.deposit_start, st));
     ws.fork_ready = !cap;
     ws.fork_capture = cid;
-    if (cap) ws.captured = true;
-    else ws.start_recorded = true;
     return SC_OK;
 }
 
@@ -585,16 +572,13 @@ int ensure_side_stream(Mesh *m)
         ctx->side = nullptr;
         return SC_ERR_DEVICE;
     }
-    if (!ws.green_done && hipEventCreateWithFlags(&ws.green_done, hipEventDisableTiming) != hipSuccess) {
+    // they order streams of this device only: released at device scope
+    constexpr unsigned kFlags = hipEventDisableTiming | hipEventReleaseToDevice;
+    if (!ws.green_done && hipEventCreateWithFlags(&ws.green_done, kFlags) != hipSuccess) {
         ws.green_done = nullptr;
         return SC_ERR_DEVICE;
     }
-    if (!ws.gf_free && hipEventCreateWithFlags(&ws.gf_free, hipEventDisableTiming) != hipSuccess) {
-        ws.gf_free = nullptr;
-        return SC_ERR_DEVICE;
-    }
-    if (!ws.deposit_start &&
-        hipEventCreateWithFlags(&ws.deposit_start, hipEventDisableTiming) != hipSuccess) {
+    if (!ws.deposit_start && hipEventCreateWithFlags(&ws.deposit_start, kFlags) != hipSuccess) {
         ws.deposit_start = nullptr;
         return SC_ERR_DEVICE;
     }
@@ -607,7 +591,6 @@ void free_workspace(Mesh *m)
     // a Green build may still be running on the side stream
     if (m->ctx && m->ctx->side) (void)hipStreamSynchronize(m->ctx->side);
     if (ws.green_done) (void)hipEventDestroy(ws.green_done);
-    if (ws.gf_free) (void)hipEventDestroy(ws.gf_free);
     if (ws.deposit_start) (void)hipEventDestroy(ws.deposit_start);
     void *ptrs[] = {ws.A, ws.B, ws.Gf, ws.Gi, ws.F, ws.R, ws.twT[0], ws.twT[1], ws.twT[2]};
     for (void *p : ptrs)
@@ -722,7 +705,6 @@ int solve_class_t(Ctx *ctx, Mesh *const *ms, int k, const double *const *lo, con
                   const double *const *dl, const double *gamma, int cath, SBunch *tab)
 {
     hipStream_t st = ctx->stream;
-    unsigned long long cid = 0;
     const int mode = cath ? kFieldCathode : kFieldFree;
     for (int i = 0; i < k; ++i)
         if (int rc = ensure_workspace(ms[i])) return rc;
@@ -769,16 +751,11 @@ int solve_class_t(Ctx *ctx, Mesh *const *ms, int k, const double *const *lo, con
         else
             launch_mix_grouped<T>(ms[0], k, tab, which, mode, 1, 3, st);
         launch_end(ctx, kid[which]);
-        if (which == 2 && !stream_capturing(st, &cid)) {
-            // a later single solve's side-stream Green build waits for this
-            for (int i = 0; i < k; ++i) {
-                Workspace &ws = ms[i]->ws;
-                if (ws.gf_free) {
-                    SC_HIP(ctx, hipEventRecord(ws.gf_free, st));
-                    ws.gf_free_recorded = true;
-                }
-            }
-        }
+    }
+    for (int i = 0; i < k; ++i) {
+        // a later build without a new deposit forks after this point
+        ms[i]->ws.fork_ready = false;
+        ms[i]->ws.fork_capture = 0;
     }
     for (int i = 0; i < k; ++i) ms[i]->ws.g_valid = false;  // the reuse cache was not kept
     SC_HIP(ctx, hipGetLastError());

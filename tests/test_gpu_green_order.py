@@ -1,0 +1,77 @@
+"""GPU: the Green-function build on the side stream never overtakes a solve that
+still reads the spectra.
+
+The build overwrites the mesh's spectra on a second stream.  It forks where the
+step's deposit started, and where no deposit came since the last solve, at the
+end of the caller's stream.  Every solve of a sequence must give the bits of the
+same solve alone on a fresh mesh, whose build has nothing to overtake.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from _common import gaussian
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+GRID = (64, 48, 64)  # spectra beyond the size that is built on the caller's stream
+N = 200_000
+
+
+def _setup(T, reuse=False):
+    import spacecharge as sc
+    x, y, z = gaussian(N, (1e-3, 1e-3, 2e-3), 21)
+    p = [torch.as_tensor(a, dtype=T, device=DEV) for a in (x, y, z + 0.02, np.full(N, 1e-15))]
+    mesh = sc.Mesh3D(GRID, *p[:3], T=T)
+    if reuse:
+        mesh.set_green_reuse(True)
+    return sc, mesh, p
+
+
+def _run(sc, mesh, kind, gamma):
+    mesh.gamma = gamma
+    if kind == "potential":
+        return sc.solve_potential(mesh).clone()
+    sc.solve(mesh, at_cathode=kind == "cathode")
+    return mesh.efield.clone()
+
+
+SEQUENCE = [("field", 1.0), ("field", 3.0), ("potential", 1.0), ("cathode", 2.0), ("field", 2.0),
+            ("field", 2.0), ("potential", 4.0), ("field", 1.0)]
+
+
+# deposits: a deposit before each solve, before the first only, or on another
+# stream than the solves
+@pytest.mark.parametrize("deposits", ["each", "first", "stream"])
+@pytest.mark.parametrize("T,reuse", [(torch.float32, False), (torch.float32, True),
+                                     (torch.float64, False)])
+def test_sequence_of_solves_equals_each_alone(T, reuse, deposits):
+    sc, mesh, p = _setup(T, reuse)
+    sc.deposit(mesh, *p)
+    torch.cuda.synchronize()
+    rho = mesh.rho.clone()
+    want = []
+    for kind, gamma in SEQUENCE:
+        _, alone, _ = _setup(T)
+        alone.rho.copy_(rho)
+        want.append(_run(sc, alone, kind, gamma))
+    torch.cuda.synchronize()
+    other = torch.cuda.Stream()
+    got = []
+    for _ in range(3):
+        for kind, gamma in SEQUENCE:
+            if deposits == "each":
+                sc.deposit(mesh, *p)
+            elif deposits == "stream":
+                other.wait_stream(torch.cuda.current_stream())
+                with torch.cuda.stream(other):
+                    sc.deposit(mesh, *p)
+                torch.cuda.current_stream().wait_stream(other)
+            mesh.rho.copy_(rho)  # Float64 deposits differ in the last bits
+            got.append(_run(sc, mesh, kind, gamma))
+    torch.cuda.synchronize()
+    for i, g in enumerate(got):
+        assert torch.equal(g, want[i % len(SEQUENCE)]), (i, SEQUENCE[i % len(SEQUENCE)])
