@@ -107,9 +107,9 @@ int sc_mesh_force_generic_transforms(sc_mesh *mesh, int enable);
  * field copy that the interpolation and its adjoint gather from.  layout 1
  * holds one padded (Ex, Ey, Ez, 0) entry per node; layout 2 packs the three
  * values of a node, so that the node pairs of a cell along x are one run of six
- * (Float64 meshes only; the library also picks it for Float32 meshes of more
- * than 8 million nodes); 0 (the default) lets the library choose: packed for
- * Float64 meshes, and no copy at all where the particles are few per node.
+ * (Float64 meshes only); 0 (the default) lets the library choose: packed for
+ * Float64 meshes and for small and very large Float32 ones, and no copy at all
+ * where the particles are few per node.
  * Results are the same bits in every layout.  Changing it synchronises the
  * context's stream and frees the current copy. */
 int sc_mesh_set_field_layout(sc_mesh *mesh, int layout);

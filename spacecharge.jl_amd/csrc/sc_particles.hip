@@ -104,12 +104,14 @@ struct V4<double> {
 // its random rows miss, in the L1 while the copy is small and in the L2 and the
 // last-level cache as it grows.  Measured (copy and gather, us), Float64, P = 1 /
 // node pairs padded to 64 bytes, an earlier layout / P = 2: 4M particles on 128^3
-// - / 231 / 173, the 2M cathode bunch on 64x64x128 - / 99 / 80, 1M on 64^3 53 / 49
-// / 38, 8M on 256^3 944 / 1243 / 750: packed for every Float64 mesh.  Float32, P =
-// 1 / 2: 128^3 104 / 119 (the 24-byte runs straddle 16 bytes), 160^3 78 / 81, 256^3
-// 504 / 437: packed beyond kPackedNodes32 nodes, where the padded copy outgrows
-// the last-level cache.
-constexpr int64_t kPackedNodes32 = 8000000;
+// - / 231 / 173, the 2M cathode bunch on 64x64x128 - / 99 / 73, 1M on 64^3 53 / 49
+// / 38, 8M on 256^3 944 / 1243 / 750: packed for every Float64 mesh.  Float32, where
+// a run of six straddles its 16-byte loads, P = 1 / 2: 2M on 64^3 48 / 44, 8M on
+// 64x64x128 174 / 155, but 4M on 128^3 104 / 108, 8M on 128x128x256 235 / 240 and
+// even between; then 2M on 160^3 78 / 75, 4M on 200^3 183 / 162, 8M on 256^3 514 /
+// 437: packed where that brings the copy near the 4 MB of an L2, and where the
+// padded copy presses on the last-level cache.
+bool packed_copy(int dtype, int64_t M) { return dtype == SC_F64 || M <= 600000 || M > 4200000; }
 
 template <typename MT>
 __device__ __forceinline__ void interleave_body(int64_t i, const MT *__restrict__ ef,
@@ -668,10 +670,9 @@ int ensure_efi(Mesh *m)
 {
     if (!m->efi) {
         const int64_t M = m->n[0] * m->n[1] * m->n[2];
-        // packed for Float64 fields and large Float32 ones (see
-        // interleave_body), unless the mesh asks for a layout
+        // the mesh's own layout, or by size
         if (m->efi_layout) m->efi_pair = m->efi_layout;
-        else m->efi_pair = m->dtype == SC_F64 || M > kPackedNodes32 ? 2 : 1;
+        else m->efi_pair = packed_copy(m->dtype, M) ? 2 : 1;
         if (hipMalloc(&m->efi, (size_t)M * (m->efi_pair == 2 ? 3 : 4) * m->dtype) != hipSuccess)
             return set_err(m->ctx, SC_ERR_NOMEM, "device allocation of the interleaved field failed");
     }
