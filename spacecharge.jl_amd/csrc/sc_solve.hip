@@ -426,7 +426,13 @@ int run_solve(Mesh *m, const double lo[3], const double hi[3], const double dl[3
     // ---- forward x, y ----
     cpx<T> *F = static_cast<cpx<T> *>(io.fwd);
     cpx<T> *B = static_cast<cpx<T> *>(io.inv);
-    if (!fast(0)) {
+    const bool plane = plane_lengths(m, d);
+    if (plane) {
+        launch_begin(ctx, K_RHO_FWD_X);
+        launch_plane<T>(m, static_cast<const T *>(io.in), F, nullptr, nullptr, 1, io.nin, false, st);
+        launch_end(ctx, K_RHO_FWD_X);
+    }
+    if (!plane && !fast(0)) {
         with_fft_elems<T>(d.Lx, [&](auto e, auto t) {
             constexpr int E = decltype(e)::value, NT = decltype(t)::value;
             const int nb = pick_nb(d.Lx, E * NT, 16);
@@ -438,7 +444,7 @@ int run_solve(Mesh *m, const double lo[3], const double hi[3], const double dl[3
             launch_end(ctx, K_RHO_FWD_X);
         });
     }
-    if (!fast(1)) {
+    if (!plane && !fast(1)) {
         with_fft_elems<T>(d.Ly, [&](auto e, auto t) {
             constexpr int E = decltype(e)::value, NT = decltype(t)::value;
             const int nb = pick_nb(d.Ly, E * NT, 16);
@@ -479,7 +485,12 @@ int run_solve(Mesh *m, const double lo[3], const double hi[3], const double dl[3
     ws.fork_ready = false;
     ws.fork_capture = 0;
     // ---- backward y, x ----
-    if (!fast(3)) {
+    if (plane) {
+        launch_begin(ctx, K_INV_X);
+        launch_plane<T>(m, nullptr, B, static_cast<T *>(io.out), nullptr, 1, io.nout, true, st);
+        launch_end(ctx, K_INV_X);
+    }
+    if (!plane && !fast(3)) {
         with_fft_elems<T>(d.Ly, [&](auto e, auto t) {
             constexpr int E = decltype(e)::value, NT = decltype(t)::value;
             const int nb = pick_nb(d.Ly, E * NT, 16);
@@ -490,7 +501,7 @@ int run_solve(Mesh *m, const double lo[3], const double hi[3], const double dl[3
             launch_end(ctx, K_INV_Y);
         });
     }
-    if (!fast(4)) {
+    if (!plane && !fast(4)) {
         with_fft_elems<T>(d.Lx, [&](auto e, auto t) {
             constexpr int E = decltype(e)::value, NT = decltype(t)::value;
             const int nb = pick_nb(d.Lx, E * NT, 16);
@@ -743,10 +754,14 @@ int solve_class_t(Ctx *ctx, Mesh *const *ms, int k, const double *const *lo, con
     build_green_grouped<T>(ms[0], k, tab, 1.0, mode, st);
     launch_end(ctx, K_GREEN_F);
     static const int kid[5] = {K_RHO_FWD_X, K_RHO_FWD_Y, K_ZCONV, K_INV_Y, K_INV_X};
+    const bool plane = plane_lengths(ms[0], d);
     for (int which = 0; which < 5; ++which) {
+        if (plane && (which == 1 || which == 3)) continue;  // part of the x pass's kernel
         launch_begin(ctx, kid[which]);
         const int L = which == 0 || which == 4 ? d.Lx : which == 2 ? d.Lz : d.Ly;
-        if (engine_of(ms[0], L, dims_padded(d)) == kPow2)
+        if (plane && which != 2)
+            launch_plane<T>(ms[0], nullptr, nullptr, nullptr, tab, k, which == 0 ? 1 : 3, which == 4, st);
+        else if (engine_of(ms[0], L, dims_padded(d)) == kPow2)
             launch_fast_grouped<T>(ms[0], k, tab, which, mode, 1, 3, st);
         else
             launch_mix_grouped<T>(ms[0], k, tab, which, mode, 1, 3, st);

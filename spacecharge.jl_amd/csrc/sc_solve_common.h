@@ -113,6 +113,24 @@ inline Engine engine_of(const Mesh *m, int L, bool padded)
     if (!padded && L >= 32 && (L & (L - 1)) == 0) return kPow2;
     return smooth_lengths(m) ? kGeneric : kMix;
 }
+// Whether the x and y passes run as one kernel per direction (sc_solve_plane.hip):
+// two short axes of any lengths up to 64, or two equal longer ones as far as the
+// plane's pencils fit a workgroup (1024 lanes, and 160 KB of LDS in Float64).  One
+// solve with its Green build, separate passes / this (us): Float32 16^3 34.6 / 26.8,
+// 32^3 36.7 / 31.1, 32x32x512 164 / 155, 50^3 47.6 / 41.9, 64^3 60.9 / 56.0, 64x64x256
+// 129 / 121, 65x65x129 90.4 / 90.0; Float64 16^3 30.6 / 26.4, 32^3 36.1 / 32.2,
+// 32x32x512 234 / 220, 50^3 56.1 / 52.8, 48x48x96 73.2 / 73.1, 48x48x256 122 / 116; and
+// two launches fewer for the host.  Meshes with smooth_lengths keep their bits, and
+// force_generic_transforms its engine.
+inline bool plane_lengths(const Mesh *m, const Dims &d)
+{
+    if (m->generic_transforms || smooth_lengths(m)) return false;
+    auto is_short = [](int L) { return L == 16 || L == 24 || L == 32 || L == 48 || L == 64; };
+    if (is_short(d.Lx) && is_short(d.Ly)) return true;
+    if (d.Lx != d.Ly) return false;
+    if (d.Lx == 128 || d.Lx == 144 || d.Lx == 160) return m->dtype == SC_F32;
+    return d.Lx == 72 || d.Lx == 80 || d.Lx == 96 || d.Lx == 100;
+}
 // true when some axis is padded beyond twice its nodes
 inline bool dims_padded(const Dims &d) { return d.nx != d.mx || d.ny != d.my || d.nz != d.mz; }
 
@@ -223,6 +241,11 @@ template <typename T>
 bool launch_fast(Mesh *m, int which, const SolveIO &io);
 template <typename T>
 bool launch_mix(Mesh *m, int which, const SolveIO &io);
+// The x and y passes of one mesh, or (tab) of nb same-shape bunches: forward from
+// `in` to `spec`, or inverse from `spec` to `out`, ncomp components.
+template <typename T>
+void launch_plane(const Mesh *m, const T *in, cpx<T> *spec, T *out, const SBunch *tab, int nb, int ncomp,
+                  bool inverse, hipStream_t st);
 
 // Grouped forms, on `st`, for nb bunches of the mesh shape of m0 whose
 // transforms run on the register engines: the Green build (field modes) of
