@@ -442,10 +442,10 @@ def kernel_bytes(name, n, grid, s, ps):
     if name == "gather_tiles":
         return tiles * 17 ** 3 * 8 + M * s
     if name == "interleave":
-        # reads the three components, writes 4 values per node, or 8 (node
-        # pairs) for Float64 fields of 64 MiB and more, as the library picks
-        pair = 2 if (s == 8 and M * 32 >= (64 << 20)) else 1
-        return 3 * M * s + 4 * pair * M * s
+        # reads the three components, writes them packed, or with a fourth value
+        # per node on middle-sized Float32 meshes, as the library picks
+        packed = s == 8 or M <= 600000 or M > 4200000
+        return 3 * M * s + (3 if packed else 4) * M * s
     if name == "interpolate":
         # positions in, fields out, and the field once (6 Np s + 3 M s)
         return 6 * n * ps + 3 * M * s
