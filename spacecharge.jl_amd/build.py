@@ -31,7 +31,7 @@ UNITS += [("sc_green.hip", f"_{k}", [f"-DSC_GREEN_PART={k}"]) for k in range(2)]
 UNITS += [("sc_solve_plane.hip", f"_{k}", [f"-DSC_PLANE_PART={k}"]) for k in range(2)]
 UNITS += [("sc_api.cpp", "", []), ("sc_particles.hip", "", []), ("sc_deposit.hip", "", []),
           ("sc_solve.hip", "", []), ("sc_solve_fast.hip", "", [])]
-HEADERS = ["sc_internal.h", "sc_fft_dev.h", "sc_fft_reg.h", "sc_fft_mix.h",
+HEADERS = ["sc_internal.h", "sc_deposit_plan.h", "sc_fft_dev.h", "sc_fft_reg.h", "sc_fft_mix.h",
            "sc_solve_common.h"]
 
 

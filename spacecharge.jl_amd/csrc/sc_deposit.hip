@@ -31,7 +31,7 @@
 //   gather_tiles   one lane per node: sum over the (up to 8) tiles whose
 //               sub-grid holds the node, in a fixed order
 //
-// Meshes of few tiles skip the binning (k_deposit_direct, direct_slices).
+// Meshes of few tiles skip the binning (k_deposit_direct, direct_most).
 //
 // A particle's eight contributions are computed exactly as in the reference
 // (same operation order, no FMA contraction); only the order of the sums
@@ -44,6 +44,7 @@
 #include <cstring>
 #include <type_traits>
 
+#include "sc_deposit_plan.h"
 #include "sc_internal.h"
 
 namespace sc {
@@ -55,20 +56,10 @@ constexpr int kSub = kTile + 1;      // nodes per sub-grid edge
 constexpr int kSubVol = kSub * kSub * kSub;
 constexpr int kRange = 4096;         // tiles per LDS histogram (one binning range)
 constexpr int kMaxTiles = 65535;     // tiles of the binned path (a grid axis of the reduction)
-constexpr int64_t kCmatBudget = (int64_t)1 << 22;  // count-matrix entries (slices x tiles)
 constexpr int kBinThreads = 256;
 constexpr int kBatch = 8;            // particles a lane loads before computing any
 // particles per deposit workgroup: 2^chunk_log2, a per-mesh setting
 // (Mesh::chunk_log2, kChunkLog2Min..kChunkLog2Max)
-constexpr int kDepThreads = 512;     // deposit workgroup size
-constexpr int kBinMaxSlices = 2048;  // binning workgroups (columns of the count matrix)
-
-// direct deposit (k_deposit_direct): most tiles, most particle-tile pairs (most
-// particles on one tile), particles per workgroup, workgroups aimed at
-constexpr int kDirectTiles = 64;
-constexpr int64_t kDirectPairs = (int64_t)4 << 20, kDirectMost = (int64_t)16 << 20;
-constexpr int kDirectLog2 = 13;
-constexpr int kDirectBlocks = 128;
 
 inline int div_up4(int a) { return (a + 3) / 4; }
 
@@ -140,13 +131,6 @@ __device__ __forceinline__ int tile_of(PT px, PT py, PT pz, const Geo &g)
     bool ext;
     return tile_of<PT, MT>(px, py, pz, g, ext);
 }
-
-// The binning workgroups split the particles into G contiguous slices of
-// `slice` particles; all three binning kernels use the same split.
-struct Split {
-    int64_t n, slice;
-    int G;
-};
 
 // Per-slice tile histogram, written as column w of the [tile][G] matrix.
 // Each lane loads kBatch particles before it computes any, so the loads of
@@ -830,7 +814,7 @@ k_gather_tiles(const double *__restrict__ partials, size_t pstride,
 // records, no tile tables.  Bound by its dependent phases (read, list, deposit,
 // store) and by the 39 KB sub-grid that each workgroup writes.  The
 // particles are read once per tile (from the L2), so the product of tiles and
-// particles bounds the range (direct_slices).
+// particles bounds the range (direct_most).
 //
 // Float32 meshes accumulate in fixed point by the binned chain's rules (the
 // scale from max|q| over all particles, Float64 in tiles that hold a particle
@@ -1090,45 +1074,13 @@ k_gather_direct(const double *__restrict__ partials, size_t pstride, const unsig
     }
 }
 
-// Slices of the direct deposit (nchan charge channels) of n particles on a mesh
-// of T tiles, or 0 where the binned chain takes it: a mesh with a deposit
-// tiling of its own, and too many particle-tile pairs.  Measured (replayed from
-// a graph, direct / binned, us), Float64: 10k particles on 16^3 7.7 / 37; 50k
-// and 200k on 32^3 (8 tiles) 19 / 38 and 27 / 43, 1M 86 / 54; 50k on 64^3 (64
-// tiles) 34 / 39, 200k 76 / 44: the two cross near 4M pairs.  Float32, with one
-// launch more: 10k on 16^3 13 / 32, 1M 25 / 50; 200k on 32^3 29 / 40; 50k on 48^3
-// (27 tiles) 37 / 35: near 1.5M pairs, kept at 2M for the three launches that it
-// saves the host.  One tile has no pairs to spare: there only the size of the
-// sub-grids ends the range.
-int direct_slices(const Mesh *m, int64_t n, int T, int nchan)
+// Slices of the direct deposit of n particles on a mesh of T tiles, or 0 where
+// the binned chain takes it: a mesh with a deposit tiling of its own, and too
+// many particle-tile pairs (direct_most).
+int direct_slices_of(const Mesh *m, int64_t n, int T, int nchan)
 {
     if (m->chunk_log2 != kChunkLog2Default || m->slice_log2 != kSliceLog2Default) return 0;
-    const int64_t most_pairs = T == 1 ? kDirectMost : (m->dtype == SC_F32 ? kDirectPairs / 2 : kDirectPairs);
-    if (T > kDirectTiles || n * T * nchan > most_pairs) return 0;
-    const int64_t per = (int64_t)1 << kDirectLog2;
-    const int64_t least = (n + per - 1) / per;  // slices of at most 2^kDirectLog2
-    const int64_t most = (n + kDepThreads - 1) / kDepThreads;
-    int64_t G = (T == 1 ? 2 : 1) * kDirectBlocks / T;
-    if (G > most) G = most;
-    if (G < least) G = least;
-    return (int)G;
-}
-
-// At most kBinMaxSlices slices of about 2^slice_log2 particles, and at
-// most kCmatBudget / ntiles (the count matrix has a row per tile).
-Split split_of(int64_t n, int slice_log2, int ntiles)
-{
-    Split sp;
-    sp.n = n;
-    const int64_t per = (int64_t)1 << slice_log2;
-    int64_t G = (n + per - 1) / per;
-    if (G > kBinMaxSlices) G = kBinMaxSlices;
-    const int64_t gmax = kCmatBudget / (ntiles > 0 ? ntiles : 1);
-    if (G > gmax) G = gmax;
-    if (G < 1) G = 1;
-    sp.G = (int)G;
-    sp.slice = (n + G - 1) / G;
-    return sp;
+    return n <= direct_most(T, m->dtype == SC_F32, nchan) ? direct_slices(n, T) : 0;
 }
 
 // Entries of each per-tile block of the counts array (totals, tile start,
@@ -1136,47 +1088,10 @@ Split split_of(int64_t n, int slice_log2, int ntiles)
 // binning range (the layout the grouped launches assume), else the tiles.
 int counts_stride(int ntiles) { return ntiles > kRange ? ntiles : kRange; }
 
-// Room for `need` chunks and sub-grids in each of nchan channel sets.
-int grow_partials(Mesh *m, int64_t need, int nchan)
-{
-    DepositBins &B = m->bins;
-    auto fail = [&]() {
-        return set_err(m->ctx, SC_ERR_NOMEM, "device allocation of the deposit bins failed");
-    };
-    const int64_t cap = B.chunk_cap > need ? B.chunk_cap : need;
-    const int sets = B.partial_sets > nchan ? B.partial_sets : nchan;
-    if (B.chunks) (void)hipFree(B.chunks);
-    if (B.partials) (void)hipFree(B.partials);
-    B.chunks = B.partials = nullptr;
-    B.chunk_cap = 0;
-    B.partial_sets = 0;
-    if (hipMalloc(&B.chunks, sizeof(int4) * cap) != hipSuccess) return fail();
-    // one sub-grid per chunk and channel, in the wider mesh type (double
-    // covers both); channel c's set starts c * cap sub-grids in
-    if (hipMalloc(&B.partials, sizeof(double) * kSubVol * (size_t)cap * sets) != hipSuccess)
-        return fail();
-    B.chunk_cap = cap;
-    B.partial_sets = sets;
-    return SC_OK;
-}
-
-int ensure_counts(Mesh *m, int ntiles)
-{
-    DepositBins &B = m->bins;
-    if (B.counts) return SC_OK;
-    // totals | tile start | first extra sub-grid slot | extrapolation flags | nchunks, pad |
-    // per-slice max|q| of up to three channels (u64 bit patterns); the direct
-    // deposit keeps its per-slice tile masks in the first blocks
-    const size_t bytes =
-        sizeof(unsigned) * (4 * (size_t)counts_stride(ntiles) + 4 + 3 * 2 * kBinMaxSlices);
-    if (hipMalloc((void **)&B.counts, bytes) != hipSuccess)
-        return set_err(m->ctx, SC_ERR_NOMEM, "device allocation of the deposit bins failed");
-    return SC_OK;
-}
-
+// Scratch of a deposit of n particles and nchan charge channels, by either path
+// (deposit_need).
 int ensure_bins(Mesh *m, int64_t n, int pdt, int ntiles, int nchan)
 {
-    const int64_t chunk = (int64_t)1 << m->chunk_log2;
     DepositBins &B = m->bins;
     const size_t rec = 4 * (size_t)pdt;
     const size_t need = (size_t)n * rec;
@@ -1190,44 +1105,48 @@ int ensure_bins(Mesh *m, int64_t n, int pdt, int ntiles, int nchan)
         if (hipMalloc(&B.sorted, need) != hipSuccess) return fail();
         B.sorted_bytes = need;
     }
-    // chunks: at most ntiles + n / chunk; sub-grid slots: below 2 ntiles + chunks
-    // (slots of the row scan's reservation order, k_bin_rowscan)
-    const int64_t maxchunks = 2 * (int64_t)ntiles + n / chunk + 1;
-    if (B.chunk_cap < maxchunks || B.partial_sets < nchan) {
-        if (int rc = grow_partials(m, maxchunks, nchan)) return rc;
+    const DepositNeed d =
+        deposit_need(n, ntiles, m->dtype == SC_F32, nchan, m->chunk_log2, m->slice_log2);
+    if (B.chunk_cap < d.chunks || B.partial_sets < nchan) {
+        const int64_t cap = B.chunk_cap > d.chunks ? B.chunk_cap : d.chunks;
+        const int sets = B.partial_sets > nchan ? B.partial_sets : nchan;
+        if (B.chunks) (void)hipFree(B.chunks);
+        if (B.partials) (void)hipFree(B.partials);
+        B.chunks = B.partials = nullptr;
+        B.chunk_cap = 0;
+        B.partial_sets = 0;
+        if (hipMalloc(&B.chunks, sizeof(int4) * cap) != hipSuccess) return fail();
+        // one sub-grid per chunk and channel, in the wider mesh type (double
+        // covers both); channel c's set starts c * cap sub-grids in
+        if (hipMalloc(&B.partials, sizeof(double) * kSubVol * (size_t)cap * sets) != hipSuccess)
+            return fail();
+        B.chunk_cap = cap;
+        B.partial_sets = sets;
     }
-    if (int rc = ensure_counts(m, ntiles)) return rc;
-    const int64_t need_cmat = (int64_t)ntiles * split_of(n, m->slice_log2, ntiles).G;
-    if (B.cmat_cap < need_cmat) {
+    if (!B.counts) {
+        // totals | tile start | first extra sub-grid slot | extrapolation flags | nchunks, pad |
+        // per-slice max|q| of up to three channels (u64 bit patterns); the direct
+        // deposit keeps its per-slice tile masks in the first blocks
+        const size_t bytes =
+            sizeof(unsigned) * (4 * (size_t)counts_stride(ntiles) + 4 + 3 * 2 * kBinMaxSlices);
+        if (hipMalloc((void **)&B.counts, bytes) != hipSuccess) return fail();
+    }
+    if (B.cmat_cap < d.cmat) {
         if (B.cmat) (void)hipFree(B.cmat);
         B.cmat = nullptr;
         B.cmat_cap = 0;
-        if (hipMalloc((void **)&B.cmat, sizeof(unsigned) * (size_t)need_cmat) != hipSuccess)
+        if (hipMalloc((void **)&B.cmat, sizeof(unsigned) * (size_t)d.cmat) != hipSuccess)
             return fail();
-        B.cmat_cap = need_cmat;
+        B.cmat_cap = d.cmat;
     }
-    return SC_OK;
-}
-
-// Scratch of the direct deposit: T G sub-grids per channel, and their flags.
-int ensure_direct(Mesh *m, int T, int G, int nchan)
-{
-    DepositBins &B = m->bins;
-    auto fail = [&]() {
-        return set_err(m->ctx, SC_ERR_NOMEM, "device allocation of the deposit bins failed");
-    };
-    if (int rc = ensure_counts(m, T)) return rc;
-    const int64_t need = (int64_t)T * G;
-    if (B.chunk_cap < need || B.partial_sets < nchan) {
-        if (int rc = grow_partials(m, need, nchan)) return rc;
-    }
-    if (B.cmat_cap < need * nchan) {
-        if (B.cmat) (void)hipFree(B.cmat);
-        B.cmat = nullptr;
-        B.cmat_cap = 0;
-        if (hipMalloc((void **)&B.cmat, sizeof(unsigned) * (size_t)(need * nchan)) != hipSuccess)
-            return fail();
-        B.cmat_cap = need * nchan;
+    // records of the further channels, for the binned chain
+    const size_t need_qs = nchan > 1 ? (size_t)2 * n * pdt : 0;
+    if (B.qs_bytes < need_qs) {
+        if (B.qs) (void)hipFree(B.qs);
+        B.qs = nullptr;
+        B.qs_bytes = 0;
+        if (hipMalloc(&B.qs, need_qs) != hipSuccess) return fail();
+        B.qs_bytes = need_qs;
     }
     return SC_OK;
 }
@@ -1473,8 +1392,8 @@ int launch_deposit_binned_multi(Mesh *m, int pdt, const void *x, const void *y, 
     }
     note_particles(m, pdt);
     const int T = g.tx * g.ty * g.tz;
-    if (const int G = direct_slices(m, n, T, nchan)) {
-        if (int rc = ensure_direct(m, T, G, nchan)) return rc;
+    if (int rc = ensure_bins(m, n, pdt, T, nchan)) return rc;
+    if (const int G = direct_slices_of(m, n, T, nchan)) {
         if (pdt == SC_F32 && m->dtype == SC_F32)
             return direct<float, float>(m, x, y, z, q, nchan, n, g, clear, out, G);
         if (pdt == SC_F64 && m->dtype == SC_F64)
@@ -1482,19 +1401,6 @@ int launch_deposit_binned_multi(Mesh *m, int pdt, const void *x, const void *y, 
         if (pdt == SC_F64 && m->dtype == SC_F32)
             return direct<double, float>(m, x, y, z, q, nchan, n, g, clear, out, G);
         return direct<float, double>(m, x, y, z, q, nchan, n, g, clear, out, G);
-    }
-    if (int rc = ensure_bins(m, n, pdt, T, nchan)) return rc;
-    if (nchan > 1) {
-        DepositBins &B = m->bins;
-        const size_t need = (size_t)2 * n * pdt;
-        if (B.qs_bytes < need) {
-            if (B.qs) (void)hipFree(B.qs);
-            B.qs = nullptr;
-            B.qs_bytes = 0;
-            if (hipMalloc(&B.qs, need) != hipSuccess)
-                return set_err(m->ctx, SC_ERR_NOMEM, "device allocation of the deposit bins failed");
-            B.qs_bytes = need;
-        }
     }
     if (pdt == SC_F32 && m->dtype == SC_F32)
         return binned<float, float>(m, x, y, z, q, nchan, n, g, clear, out);
