@@ -691,6 +691,20 @@ int ensure_efi(Mesh *m)
     return SC_OK;
 }
 
+// Makes the field copy of a mesh that gathers without one, ahead of a call that
+// needs it (more particles, the adjoint): that call may be under capture, where
+// nothing can be allocated, and one eager call is to prepare it.  Nothing is lost
+// where the memory is short.
+void reserve_efi(Mesh *m)
+{
+    unsigned long long id = 0;
+    if (m->efi || stream_capturing(m->ctx->stream, &id)) return;
+    if (ensure_efi(m) != SC_OK) {
+        m->efi = nullptr;
+        (void)hipGetLastError();
+    }
+}
+
 }  // namespace
 
 int launch_clear(Ctx *ctx, void *p, int64_t bytes)
@@ -787,6 +801,7 @@ int launch_interp(Mesh *m, int pdt, const void *x, const void *y, const void *z,
 {
     if (n <= 0) return SC_OK;
     if (gather_direct(m, n)) {
+        reserve_efi(m);
         launch_begin(m->ctx, K_INTERP);
         if (pdt == SC_F32 && m->dtype == SC_F32) itp_soa<float, float>(m, x, y, z, n, lo, dl, Ex, Ey, Ez);
         else if (pdt == SC_F64 && m->dtype == SC_F64)
@@ -1061,9 +1076,10 @@ int launch_interp_grouped(Ctx *ctx, Mesh *const *ms, int nb, int pdt, const void
         if (blocks > 0x7fffffffLL || (M + 255) / 256 > 0x7fffffffLL) return SC_ERR_UNSUPPORTED;
     }
     if (int rc = ensure_group_table(ctx, group_table_bytes())) return rc;
-    for (int b = 0; b < nb; ++b)
-        if (!gather_direct(ms[b], n[b]))
-            if (int rc = ensure_efi(ms[b])) return rc;
+    for (int b = 0; b < nb; ++b) {
+        if (gather_direct(ms[b], n[b])) reserve_efi(ms[b]);
+        else if (int rc = ensure_efi(ms[b])) return rc;
+    }
     ITable *T = static_cast<ITable *>(ctx->gtable);
     unsigned total[kIPhases] = {};
     IStore s;

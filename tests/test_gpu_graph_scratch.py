@@ -112,3 +112,38 @@ def test_captured_cotangent_deposit_with_a_tiling_set_after_the_eager_one(T):
         assert _same(out, got)
         for c in g:
             c.mul_(0.5)
+
+
+# few: gathered without the field copy
+@pytest.mark.parametrize("T", [torch.float32, torch.float64])
+@pytest.mark.parametrize("call", ["single", "batched", "adjoint"])
+def test_captured_interpolation_after_an_eager_one_of_few_particles(T, call):
+    import spacecharge as sc
+    many = _bunch(300_000, 5, T)[:3]
+    few = [a[:1000].clone() for a in many]
+    mesh, ref = (sc.Mesh3D((32, 32, 32), *many, T=T) for _ in range(2))
+    g = torch.Generator(device=DEV).manual_seed(2)
+    ef = torch.randn(mesh.efield.shape, generator=g, device=DEV, dtype=T)
+    cot = [torch.randn(many[0].shape, generator=g, device=DEV, dtype=T) for _ in range(3)]
+
+    def run(m, p):
+        if call == "batched":
+            return sc.interpolate_batched([m], *[[a] for a in p])[0]
+        if call == "adjoint" and len(p[0]) > 1000:
+            return sc.interpolate_adjoint(m, *p, *cot)[1:]
+        return sc.interpolate_field(m, *p)
+
+    if call == "adjoint":  # its deposit's scratch
+        sc.interpolate_adjoint(mesh, *many, *cot, positions=False)
+    for m in (mesh, ref):
+        m.efield.copy_(ef)
+    run(mesh, few)
+    graph, out = _capture(lambda: run(mesh, many))
+    for rep in range(2):
+        graph.replay()
+        want = run(ref, many)
+        torch.cuda.synchronize()
+        for a, b in zip(out, want):
+            assert torch.equal(a, b)
+        for m in (mesh, ref):
+            m.efield.mul_(0.5)
