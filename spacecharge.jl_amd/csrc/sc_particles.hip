@@ -658,24 +658,23 @@ void itp_vjp(Mesh *m, const void *x, const void *y, const void *z, int64_t n, co
 }
 
 // Whether the interpolation of n particles gathers straight from efield: the
-// interleaved copy costs a launch and a pass over all M nodes, the direct
-// gather two to three times the cache lines per particle, so few particles per
-// node go direct; the larger the field, the sooner its lines miss the caches.
-// Measured, direct / interleaved (us), Float32: 200k on 128^3 (0.10 per node) 17 /
-// 21, 500k (0.24) 31 / 28; 50k on 32^3 4.9 / 7.1, 200k on 64^3 14 / 13; 500k on 256^3
-// (0.03) 80 / 100, 1M (0.06) 155 / 125.  Float64: 500k on 128^3 (0.24) 44 / 45, 1M 81 /
-// 66; 200k on 32^3 12 / 12, 500k 22.5 / 18; on 160^3 500k (0.12) 56 / 62, 1M 100 / 86;
-// on 256^3 1M (0.06) 197 / 230, 2M 381 / 304.  A forced layout keeps its copy.
+// interleaved copy costs a launch and a pass over all M nodes, the direct gather
+// two to three times the cache lines per particle.  Particles spread over the
+// whole mesh miss most, so the line lies where these break even; those of a core
+// (rms a tenth of the mesh) would gain to twice the count.  Up to 200^3 nodes they
+// break even at about 100k particles whatever the mesh, beyond that the copy's
+// pass grows.  Measured, uniform particles, direct / copy (us), Float32: 100k on
+// 32^3 7.0 / 7.1, on 64^3 7.7 / 11.8, on 128^3 20.5 / 20.0 (core 8.9 / 16.1), 200k
+// on 128^3 39.8 / 29.1; 167k on 200^3 39 / 40, 350k on 256^3 82 / 97, 524k 122 / 106.
+// Float64: 100k on 32^3 7.7 / 8.7, on 64^3 12.7 / 17.6, on 100^3 20.9 / 21.0, 262k
+// on 128^3 58 / 42; 171k on 160^3 41 / 44, 333k on 200^3 83 / 103, 699k on 256^3
+// 171 / 212, 1.05M 255 / 244.  A forced layout keeps its copy.
 bool gather_direct(const Mesh *m, int64_t n)
 {
     if (m->efi_layout) return false;
     const int64_t M = m->n[0] * m->n[1] * m->n[2];
-    if (m->dtype == SC_F32) {
-        const int64_t few = M > 6000000 ? M / 20 : M / 6;
-        return n <= (few > 131072 ? few : 131072);
-    }
-    const int64_t few = M > 6000000 ? M / 12 : M > 3000000 ? M / 6 : M / 3;
-    return n <= (few > 200000 ? few : 200000);
+    const int64_t few = M / (m->dtype == SC_F32 ? 48 : 24);
+    return n <= (few > 100000 ? few : 100000);
 }
 
 int ensure_efi(Mesh *m)
