@@ -10,10 +10,9 @@ constexpr int kBinMaxSlices = 2048;  // binning workgroups (columns of the count
 constexpr int64_t kCmatBudget = (int64_t)1 << 22;  // count-matrix entries (slices x tiles)
 constexpr int kDepThreads = 512;     // deposit workgroup size
 
-// direct deposit (k_deposit_direct): most tiles, most particle-tile pairs (most
-// particles on one tile), particles per workgroup, workgroups aimed at
+// direct deposit (k_deposit_direct): most tiles, particles per workgroup,
+// workgroups aimed at
 constexpr int kDirectTiles = 64;
-constexpr int64_t kDirectPairs = (int64_t)4 << 20, kDirectMost = (int64_t)16 << 20;
 constexpr int kDirectLog2 = 13;
 constexpr int kDirectBlocks = 128;
 
@@ -42,17 +41,28 @@ inline Split split_of(int64_t n, int slice_log2, int ntiles)
 }
 
 // Most particles that the direct deposit takes on a mesh of T tiles (0: none),
-// f32 the mesh type, nchan charge channels.  Measured (replayed from
-// a graph, direct / binned, us), Float64: 10k particles on 16^3 7.7 / 37; 50k
-// and 200k on 32^3 (8 tiles) 19 / 38 and 27 / 43, 1M 86 / 54; 50k on 64^3 (64
-// tiles) 34 / 39, 200k 76 / 44: the two cross near 4M pairs.  Float32, with one
-// launch more: 10k on 16^3 13 / 32, 1M 25 / 50; 200k on 32^3 29 / 40; 50k on 48^3
-// (27 tiles) 37 / 35: near 1.5M pairs, kept at 2M for the three launches that it
-// saves the host.  One tile has no pairs to spare: there only the size of the
-// sub-grids ends the range.
+// f32 the mesh type, nchan charge channels.  Its cost grows with the particle-tile
+// pairs and with the sub-grids, the binned chain's hardly; particles that fill
+// the mesh are the binned chain's best case, so the line lies below where those
+// break even.  Measured (replayed from a graph, uniform particles, direct / binned,
+// us), Float64: 10k on 16^3 7.7 / 37; 8 tiles, 262k (2M pairs) 27.6 / 48.7, 524k 37 /
+// 51, 734k 67 / 52; 27 tiles, 155k (4M pairs) 41.5 / 42.9, 217k 49.5 / 48; 64 tiles,
+// 33k (2M pairs) 29.6 / 35.7, 46k 36.1 / 36.2, 66k 49.7 / 36.9.  Float32, with one
+// launch more and a cheaper chain: 10k on 16^3 13 / 32; 8 tiles, 262k 31 / 41, 524k
+// 40 / 45, 734k 60 / 46; 27 tiles, 54k (1.4M pairs) 27.6 / 32, 78k (2M) 38 / 33; 64
+// tiles, 23k (1.4M) 31.5 / 32.6, 46k 40 / 33.  One tile has no pairs to spare: there
+// only the size of the sub-grids ends the range.  Three channels triple the
+// sub-grids and share one binning: 4k on 64 tiles 50 / 39 in Float32, 44.7 / 43.2 in
+// Float64, 9k on 27 tiles 35.8 / 33.9 in Float32; Float64 on 4 tiles, 245k (2.8M) 35 /
+// 53, 350k 57 / 52.
 inline int64_t direct_most(int T, bool f32, int nchan)
 {
-    const int64_t pairs = T == 1 ? kDirectMost : (f32 ? kDirectPairs / 2 : kDirectPairs);
+    constexpr int64_t k = (int64_t)1 << 20;
+    const int64_t pairs = T == 1 ? 16 * k : f32 ? (T <= 8 ? 2 * k : 7 * k / 5) : T <= 32 ? 4 * k : 5 * k / 2;
+    if (nchan > 1 && T > 1) {
+        if (T > (f32 ? 8 : 32)) return 0;
+        if (pairs > 3 * k) return 3 * k / ((int64_t)T * nchan);
+    }
     return T > kDirectTiles ? 0 : pairs / ((int64_t)T * nchan);
 }
 

@@ -37,3 +37,43 @@ def test_field_copy_of_the_interpolation(T, grid, few, many):
         assert _launched(lambda: sc.interpolate_field(mesh, *p), "interleave") == (n == many), n
         for a, b in zip(sc.interpolate_field(mesh, *p), sc.interpolate_field(copied, *p)):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("T,grid,few,many", [
+    (torch.float32, (16, 16, 16), 1_000_000, 17_000_000), (torch.float32, (32, 32, 32), 262_144, 734_000),
+    (torch.float32, (48, 48, 48), 54_370, 77_672), (torch.float32, (64, 64, 64), 22_937, 32_768),
+    (torch.float64, (32, 32, 32), 524_288, 734_000), (torch.float64, (48, 48, 48), 155_344, 217_482),
+    (torch.float64, (64, 64, 64), 40_960, 65_536), (torch.float64, (65, 65, 81), 20_000, 40_000)])
+def test_binning_of_the_deposit(T, grid, few, many):
+    import spacecharge as sc
+    mesh, binned = (sc.Mesh3D(grid, (-1.0,) * 3, (1.0,) * 3, T=T) for _ in range(2))
+    binned.set_deposit_tiling(13, 11)
+    tiles = 1
+    for n in grid:
+        tiles *= (n + 14) // 16
+    for n in (few, many):
+        p = _uniform(n, T, 4)
+        # (beyond 64 tiles every count is binned)
+        assert _launched(lambda: sc.deposit(mesh, *p), "bin_scatter") == (n == many or tiles > 64), n
+        sc.deposit(binned, *p)
+        err = float((mesh.rho - binned.rho).double().norm() / binned.rho.double().norm())
+        assert err <= (1e-6 if T == torch.float32 else 1e-13)
+
+
+@pytest.mark.parametrize("T,grid,few,many", [
+    (torch.float32, (32, 32, 32), 87_381, 174_762), (torch.float32, (48, 48, 48), 0, 9061),
+    (torch.float64, (33, 33, 17), 244_667, 349_525), (torch.float64, (64, 64, 64), 0, 3822)])
+def test_binning_of_the_cotangent_deposit(T, grid, few, many):
+    import spacecharge as sc
+    mesh, binned = (sc.Mesh3D(grid, (-1.0,) * 3, (1.0,) * 3, T=T) for _ in range(2))
+    binned.set_deposit_tiling(13, 11)
+    for n in (few, many):
+        if not n:
+            continue
+        p = _uniform(n, T, 6)
+        got = []
+        assert _launched(lambda: got.append(sc.interpolate_adjoint(mesh, *p, positions=False)[0]),
+                         "bin_scatter") == (n == many), n
+        want = sc.interpolate_adjoint(binned, *p, positions=False)[0]
+        err = float((got[0] - want).double().norm() / want.double().norm())
+        assert err <= (1e-6 if T == torch.float32 else 1e-13)
