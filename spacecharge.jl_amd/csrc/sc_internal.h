@@ -186,12 +186,16 @@ struct Workspace {
     // (latency bound) rather than the previous step's interpolation.
     // fork_ready: recorded by an eager deposit, and no solve of this mesh has
     // been launched since (its z convolution reads the spectra that the build
-    // writes); fork_capture: the id of the capture whose deposit recorded the
-    // event, likewise (0: none).  A build with no usable record forks from the
-    // end of the stream.
+    // writes) nor device-resident bounds computed (the build reads them);
+    // fork_capture: the id of the capture whose deposit recorded the event,
+    // likewise (0: none).  A build with no usable record forks from the end of
+    // the stream.  captured: a capture has solved on this mesh; its replays,
+    // which may come between an eager deposit and its solve, clear no mark, so
+    // eager builds then always fork from the end.
     hipEvent_t deposit_start = nullptr;
     bool fork_ready = false;
     unsigned long long fork_capture = 0;
+    bool captured = false;
     // cached Green key for the opt-in reuse
     bool g_valid = false;
     double g_key[6] = {};

@@ -921,6 +921,10 @@ int launch_bounds_geom(Mesh *m, int pdt, const void *x, const void *y, const voi
         m->geom = nullptr;
         return set_err(ctx, SC_ERR_NOMEM, "device allocation of the mesh geometry failed");
     }
+    // a Green build that forked at an earlier deposit would read the geometry
+    // while it is written
+    m->ws.fork_ready = false;
+    m->ws.fork_capture = 0;
     int64_t nblk = 0;
     const BoundsGeom bg{m->geom, pdt, m->dtype, {(long long)m->n[0], (long long)m->n[1], (long long)m->n[2]}};
     if (int rc = reduce_extrema(ctx, pdt, x, y, z, n, &nblk, bg)) return rc;

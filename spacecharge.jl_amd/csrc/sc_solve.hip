@@ -386,19 +386,22 @@ int run_solve(Mesh *m, const double lo[3], const double hi[3], const double dl[3
     // exist already (no stream is created while capturing).
     unsigned long long cid = 0;
     const bool cap = stream_capturing(st, &cid);
+    if (cap) ws.captured = true;
     bool overlap = false;
     if (!reuse) {
         overlap = !ctx->in_batch && !green_small(d, sizeof(T), cath) &&
                   (cap ? ctx->side && ws.green_done && ws.deposit_start : ensure_side_stream(m) == SC_OK);
         if (overlap) {
             // the build forks where this step's deposit started (recorded by
-            // a deposit of this capture, or by an eager deposit, and no solve
-            // launched since), else at the current end of `st`.  Both lie after
-            // the last z convolution that reads this mesh's Green spectra: an
-            // event of its own after each of those, for builds that fork
-            // further back, cost 5.5 us of idle device and 3 us of host time
-            // per solve
-            const bool from_deposit = cap ? ws.fork_capture == cid : ws.fork_ready;
+            // a deposit of this capture, or by an eager deposit), if no solve
+            // has been launched since and no bounds (launch_bounds_geom), which
+            // the build reads; else at the current end of `st`.  Both lie after
+            // the last z convolution that reads this mesh's Green spectra, and
+            // after the bounds: an event of its own after each convolution, for
+            // builds that fork further back, cost 5.5 us of idle device and 3 us
+            // of host time per solve.  A replayed graph leaves no trace here, so
+            // a mesh that a capture has solved on forks its eager builds at the end
+            const bool from_deposit = cap ? ws.fork_capture == cid : ws.fork_ready && !ws.captured;
             if (!from_deposit) SC_HIP(ctx, hipEventRecord(ws.deposit_start, st));
             SC_HIP(ctx, hipStreamWaitEvent(ctx->side, ws.deposit_start, 0));
             ctx->stream = ctx->side;  // the build launches (and times) on ctx->stream
@@ -767,7 +770,10 @@ int solve_class_t(Ctx *ctx, Mesh *const *ms, int k, const double *const *lo, con
             launch_mix_grouped<T>(ms[0], k, tab, which, mode, 1, 3, st);
         launch_end(ctx, kid[which]);
     }
+    unsigned long long cid = 0;
+    const bool cap = stream_capturing(st, &cid);
     for (int i = 0; i < k; ++i) {
+        if (cap) ms[i]->ws.captured = true;
         // a later build without a new deposit forks after this point
         ms[i]->ws.fork_ready = false;
         ms[i]->ws.fork_capture = 0;

@@ -75,3 +75,76 @@ def test_sequence_of_solves_equals_each_alone(T, reuse, deposits):
     torch.cuda.synchronize()
     for i, g in enumerate(got):
         assert torch.equal(g, want[i % len(SEQUENCE)]), (i, SEQUENCE[i % len(SEQUENCE)])
+
+
+# The next two read or write the spectra or the geometry beside the kernels that use
+# them if the build forks at the deposit.
+
+
+@pytest.mark.parametrize("T", [torch.float32, torch.float64])
+def test_bounds_between_deposit_and_solve(T):
+    """Device-resident bounds computed after the deposit are those that the solve uses."""
+    sc, mesh, p = _setup(T)
+    sc.deposit(mesh, *p)
+    torch.cuda.synchronize()
+    rho = mesh.rho.clone()
+    want, got = [], []
+    for rep in range(4):
+        x, y, z = (a * (1.0 + 0.25 * rep) for a in p[:3])
+        _, alone, _ = _setup(T)
+        alone.update_bounds(x, y, z)
+        alone.rho.copy_(rho)
+        torch.cuda.synchronize()
+        want.append(_run(sc, alone, "cathode" if rep % 2 else "field", 2.0))
+        torch.cuda.synchronize()
+    for rep in range(4):
+        x, y, z = (a * (1.0 + 0.25 * rep) for a in p[:3])
+        sc.deposit(mesh, *p)
+        mesh.update_bounds(x, y, z)
+        mesh.rho.copy_(rho)
+        got.append(_run(sc, mesh, "cathode" if rep % 2 else "field", 2.0))
+    torch.cuda.synchronize()
+    for rep in range(4):
+        assert torch.equal(got[rep], want[rep]), rep
+
+
+@pytest.mark.parametrize("T", [torch.float32, torch.float64])
+@pytest.mark.parametrize("batched", [False, True])
+def test_replay_between_deposit_and_solve(T, batched):
+    """A captured step replayed between an eager deposit and its solve."""
+    sc, mesh, p = _setup(T)
+    other = _setup(T)[1]
+
+    def captured():
+        mesh.gamma = 3.0
+        sc.deposit(mesh, *p)
+        mesh.rho.copy_(rho)
+        if batched:
+            sc.solve_batched([mesh, other])
+        else:
+            sc.solve(mesh)
+        return mesh.efield.clone()
+
+    sc.deposit(mesh, *p)
+    torch.cuda.synchronize()
+    rho = mesh.rho.clone()
+    other.rho.copy_(rho)
+    want = []
+    for gamma in (3.0, 1.0):
+        _, alone, _ = _setup(T)
+        alone.rho.copy_(rho)
+        want.append(_run(sc, alone, "field", gamma))
+    for _ in range(2):
+        captured()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = captured()
+    for rep in range(4):
+        sc.deposit(mesh, *p)
+        graph.replay()
+        mesh.rho.copy_(rho)
+        got = _run(sc, mesh, "field", 1.0)
+        torch.cuda.synchronize()
+        assert torch.equal(out, want[0]), rep
+        assert torch.equal(got, want[1]), rep
