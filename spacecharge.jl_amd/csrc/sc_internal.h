@@ -186,16 +186,21 @@ struct Workspace {
     // (latency bound) rather than the previous step's interpolation.
     // fork_ready: recorded by an eager deposit, and no solve of this mesh has
     // been launched since (its z convolution reads the spectra that the build
-    // writes) nor device-resident bounds computed (the build reads them);
+    // writes) nor device-resident bounds computed (the build reads them); or
+    // recorded after the z convolution of the last solve, where led < 2;
     // fork_capture: the id of the capture whose deposit recorded the event,
     // likewise (0: none).  A build with no usable record forks from the end of
     // the stream.  captured: a capture has solved on this mesh; its replays,
     // which may come between an eager deposit and its solve, clear no mark, so
     // eager builds then always fork from the end.
+    // deposited: a deposit since the last solve; led: solves behind a deposit
+    // since the last solve without one (2: two or more).
     hipEvent_t deposit_start = nullptr;
     bool fork_ready = false;
     unsigned long long fork_capture = 0;
     bool captured = false;
+    bool deposited = false;
+    int led = 2;
     // cached Green key for the opt-in reuse
     bool g_valid = false;
     double g_key[6] = {};

@@ -387,6 +387,8 @@ int run_solve(Mesh *m, const double lo[3], const double hi[3], const double dl[3
     unsigned long long cid = 0;
     const bool cap = stream_capturing(st, &cid);
     if (cap) ws.captured = true;
+    ws.led = !ws.deposited ? 0 : ws.led < 2 ? ws.led + 1 : 2;
+    ws.deposited = false;
     bool overlap = false;
     if (!reuse) {
         overlap = !ctx->in_batch && !green_small(d, sizeof(T), cath) &&
@@ -484,9 +486,13 @@ int run_solve(Mesh *m, const double lo[3], const double hi[3], const double dl[3
             launch_end(ctx, K_ZCONV);
         });
     }
-    // a later build without a new deposit forks after this point
-    ws.fork_ready = false;
+    // a later build without a new deposit forks after this point: where the
+    // stream ends then, or, on a mesh that was just solved without one, here,
+    // so that it runs beside the backward passes (a loop of solves, 128^3
+    // Float32 207 -> 192 us each; deposit, field and potential 361 -> 340)
     ws.fork_capture = 0;
+    ws.fork_ready = overlap && ws.led < 2 && !cap && !ws.captured;
+    if (ws.fork_ready) SC_HIP(ctx, hipEventRecord(ws.deposit_start, st));
     // ---- backward y, x ----
     if (plane) {
         launch_begin(ctx, K_INV_X);
@@ -568,6 +574,7 @@ bool stream_capturing(hipStream_t st, unsigned long long *id)
 int mark_deposit_start(Mesh *m)
 {
     Workspace &ws = m->ws;
+    ws.deposited = true;
     if (!ws.deposit_start) return SC_OK;
     hipStream_t st = m->ctx->stream;
     unsigned long long cid = 0;
@@ -775,6 +782,7 @@ int solve_class_t(Ctx *ctx, Mesh *const *ms, int k, const double *const *lo, con
     for (int i = 0; i < k; ++i) {
         if (cap) ms[i]->ws.captured = true;
         // a later build without a new deposit forks after this point
+        ms[i]->ws.deposited = false;
         ms[i]->ws.fork_ready = false;
         ms[i]->ws.fork_capture = 0;
     }
