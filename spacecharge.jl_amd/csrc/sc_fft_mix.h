@@ -17,7 +17,8 @@
 //
 // The lengths (SC_MIX_LENGTHS) are even, at most 512, and split into passes
 // whose radices divide one E of at most 20 values; axes of at most 256 nodes
-// are transformed at the next of them (transform_half in sc_solve_common.h).
+// are transformed at the next of them (transform_half, padding_pays in
+// sc_solve_common.h).
 // Radix-20 lanes (200 points as 20 x 10) took 20-40% longer than radix-10
 // ones (10 x 10 x 2) in every pass of a 100^3 Float32 solve: the shorter
 // lanes' third pass costs less than their occupancy gains.

@@ -48,7 +48,9 @@ inline bool reg_length(int L)
 // widest (one solve, generic at 2n's own length -> register: 201^3, 402 -> 512
 // points, 2994 -> 1531 us in Float32 and 4748 -> 2584 us in Float64; 101^3,
 // 210 -> 256, 386 -> 162 and 549 -> 269 us; 161^3 Float64 with the cathode,
-// 324 -> 384, 3377 -> 2861 us).
+// 324 -> 384, 3377 -> 2861 us); the spectra and the Green scratch grow with the
+// padding, at the worst (201^3 at 256 for 210) to 1.8 times the bytes.  Not on every
+// mesh of a longer axis (padding_pays).
 inline int transform_half(int n, bool smooth)
 {
     int t = n;
@@ -58,6 +60,31 @@ inline int transform_half(int n, bool smooth)
     }
     while (!smooth7(2 * t)) ++t;
     return t;
+}
+
+// Whether a mesh of an axis beyond the register lengths along z pads x and y to
+// them.  The z convolution and the z pass of the Green build stay on the generic
+// engine there, over more pencils, r times as many; the x and y passes gain
+// less than that costs where r is large, the more so the longer z is and the more
+// passes are generic anyway.  One solve, free / cathode (us), 7-smooth -> register
+// lengths: Float64 131x131x300 (r = 1.14) 3158 / 6272 -> 2379 / 5142, 101x129x300
+// (1.30) 2450 / 4821 -> 2112 / 4558, but 81x81x300 (1.40) 1059 / 2129 -> 1110 / 2275,
+// 101x101x1024 (1.49) 8344 / 13959 -> 9976 / 16913, 64x101x600 (1.22) 2517 / 4135 ->
+// 2581 / 4293, 201x300x300 (1.22, two generic axes) 12899 / 23771 -> 13378 / 25012;
+// Float32 81x81x300 688 / 1248 -> 579 / 1090, 101x101x400 (1.49) 1618 / 2889 -> 1547 /
+// 2700, but 51x51x600 (1.40) 717 / 1450 -> 726 / 1545, 101x101x1024 4673 / 9451 -> 4844 /
+// 10125.  With z on a register engine padding always gained (300x201x201 Float64
+// 7103 / 12303 -> 4674 / 10224).
+inline bool padding_pays(const Mesh *m)
+{
+    const int nx = (int)m->n[0], ny = (int)m->n[1], nz = (int)m->n[2];
+    if (2 * nz <= kMixMaxLength) return true;
+    const double r = (double)transform_half(nx, false) * transform_half(ny, false) /
+                     ((double)transform_half(nx, true) * transform_half(ny, true));
+    const bool far = 2 * nz >= 2 * kMixMaxLength;  // a z axis of 512 nodes and more
+    if (m->dtype == SC_F32) return !far || r <= 4.0 / 3.0;
+    if (2 * nx > kMixMaxLength || 2 * ny > kMixMaxLength) return r <= 1.1;
+    return r <= (far ? 1.2 : 4.0 / 3.0);
 }
 
 // Float32 meshes that carry Float64 particles keep the plain 7-smooth lengths
@@ -90,7 +117,7 @@ inline Dims make_dims(const Mesh *m)
     d.mx = (int)m->n[0];
     d.my = (int)m->n[1];
     d.mz = (int)m->n[2];
-    const bool smooth = smooth_lengths(m);
+    const bool smooth = smooth_lengths(m) || !padding_pays(m);
     d.nx = transform_half(d.mx, smooth);
     d.ny = transform_half(d.my, smooth);
     d.nz = transform_half(d.mz, smooth);

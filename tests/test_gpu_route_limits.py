@@ -77,3 +77,39 @@ def test_binning_of_the_cotangent_deposit(T, grid, few, many):
         want = sc.interpolate_adjoint(binned, *p, positions=False)[0]
         err = float((got[0] - want).double().norm() / want.double().norm())
         assert err <= (1e-6 if T == torch.float32 else 1e-13)
+
+
+def _workspace(halves, grid, size):
+    """Bytes of the solver's workspace for these transform half-lengths."""
+    (hx, hy, hz), (_, _, mz) = halves, grid
+    kp = (hx + 1 + 31) // 32 * 32
+    spec, gf, gi = mz * 2 * hy * kp, (hz + 1) * (hy + 1) * kp, 2 * hz * (hy + 1) * kp
+    fn, rn = (hx + 1) * (hy + 1) * (3 * hz + 1), (hy + 1) * kp * (3 * hz - 1)
+    return 8 * size * spec + 3 * size * gf + 6 * size * gi + 24 * fn + 3 * size * rn
+
+
+# z beyond the register lengths: x and y padded to them only where that is faster
+@pytest.mark.parametrize("T,grid,halves", [
+    (torch.float64, (51, 51, 300), (54, 54, 300)), (torch.float64, (33, 47, 300), (36, 48, 300)),
+    (torch.float64, (33, 51, 600), (35, 54, 600)), (torch.float64, (26, 257, 257), (27, 270, 270)),
+    (torch.float64, (257, 26, 26), (270, 32, 32)), (torch.float32, (51, 51, 300), (64, 64, 300)),
+    (torch.float32, (51, 51, 600), (54, 54, 600)), (torch.float32, (33, 47, 600), (36, 48, 600))])
+def test_padding_of_the_transforms(T, grid, halves):
+    import spacecharge as sc
+    g = torch.Generator(device=DEV).manual_seed(3)
+    rho = torch.rand(grid, generator=g, device=DEV, dtype=T)
+    out = []
+    for generic in (False, True):
+        m = sc.Mesh3D(grid, (-1e-3, -1e-3, 1e-4), (1e-3, 1.2e-3, 2e-3), T=T, gamma=1.5)
+        if generic:
+            m.force_generic_transforms()
+        m.rho.copy_(rho)
+        for cath in (False, True):
+            sc.solve(m, at_cathode=cath)
+            out.append(m.efield.double())
+        assert m.workspace_bytes == _workspace(halves, grid, T.itemsize)
+        del m
+    for a, b in ((out[0], out[2]), (out[1], out[3])):
+        for c in range(3):
+            d = (a[..., c] - b[..., c]).norm() / b[..., c].norm()
+            assert float(d) <= (1e-5 if T == torch.float32 else 1e-12)
