@@ -529,6 +529,7 @@ int sc_clear_mesh(sc_mesh *mesh)
     if (!mesh) return set_err(nullptr, SC_ERR_INVALID, "mesh is NULL");
     Mesh &M = mesh->m;
     if (int rc = check_dev(M.ctx)) return rc;
+    M.wide_rho = false;
     return launch_clear(M.ctx, M.rho, M.n[0] * M.n[1] * M.n[2] * M.dtype);
 }
 

@@ -1390,7 +1390,6 @@ int launch_deposit_binned_multi(Mesh *m, int pdt, const void *x, const void *y, 
         g.lo[a] = lo ? lo[a] : 0.0;
         g.dl[a] = lo ? dl[a] : 1.0;
     }
-    note_particles(m, pdt);
     const int T = g.tx * g.ty * g.tz;
     if (int rc = ensure_bins(m, n, pdt, T, nchan)) return rc;
     if (const int G = direct_slices_of(m, n, T, nchan)) {
@@ -1641,7 +1640,7 @@ int launch_deposit_grouped(Ctx *ctx, Mesh *const *ms, int nb, int pdt, const voi
     if (int rc = ensure_group_table(ctx, group_table_bytes())) return rc;
     for (int b = 0; b < nb; ++b)
         if (int rc = ensure_bins(ms[b], n[b], pdt, geos[b].tx * geos[b].ty * geos[b].tz, 1)) return rc;
-    for (int b = 0; b < nb; ++b) note_particles(ms[b], pdt);
+    for (int b = 0; b < nb; ++b) note_charges(ms[b], pdt, n[b], clear);
     // where each mesh's deposit starts on the stream (a later solve's Green
     // build on the side stream waits for it, as after launch_deposit)
     for (int b = 0; b < nb; ++b)

@@ -1266,7 +1266,7 @@ constexpr int kFxBlocks = 512;
 // last-level cache (8M particles on 256^3 Float32 2607 -> 2548 us; 256^3 Float64
 // build 1027 -> 930).  Between, beside the deposit, its longer arithmetic costs
 // more than the traffic it saves (128^3: 401 -> 408 us Float32, 688 -> 696 Float64;
-// 100^3 207 -> 210).  Meshes with smooth_lengths keep the separate kernels' bits.
+// 100^3 207 -> 210).  Solves with smooth_lengths keep the separate kernels' bits.
 bool green_fused(const Mesh *m, const Dims &d, size_t size, int cath)
 {
     if (smooth_lengths(m) || engine_of(m, d.Lx, false) == kGeneric) return false;

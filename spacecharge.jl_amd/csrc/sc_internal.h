@@ -159,7 +159,6 @@ constexpr int kChunkLog2Default = 13, kSliceLog2Default = 12;
 // Device workspace of one mesh (lazy, like src/mesh.jl:49-72).
 struct Workspace {
     bool ready = false;
-    bool smooth = false;  // transform lengths: see smooth_lengths (fixed when the workspace is made)
     int dtype = 0;
     int64_t bytes = 0;
     // spectra in the mesh type T: A = rho after the x and y transforms,
@@ -175,7 +174,11 @@ struct Workspace {
     // rows (T).
     double *F = nullptr;
     void *R = nullptr;
-    // twiddle tables in T for the lengths 2nx, 2ny, 2nz
+    // twiddle tables in T and plans for the lengths 2nx, 2ny, 2nz: of each of
+    // the two sets of lengths that a Float32 mesh has (smooth_lengths; one table
+    // where they agree), and of the set that the current solve takes
+    void *twSet[2][3] = {};
+    FftPlan planSet[2][3];
     void *twT[3] = {nullptr, nullptr, nullptr};
     FftPlan plan[3];
     // ordering of the Green build on the side stream: green_done after the
@@ -203,7 +206,7 @@ struct Workspace {
     int led = 2;
     // cached Green key for the opt-in reuse
     bool g_valid = false;
-    double g_key[6] = {};
+    double g_key[7] = {};
     int g_cath = 0;  // solve mode the cached spectra were built for
 };
 
@@ -231,7 +234,10 @@ struct Mesh {
     bool owns = false;
     bool green_reuse = false;
     bool generic_transforms = false;  // diagnostic: skip the register-resident engine
-    bool f64_particles = false;       // a Float32 mesh that Float64 particles were deposited on
+    // a Float32 mesh: Float64 particles went into rho since it was last cleared,
+    // or into the last cotangent deposit; smooth: the lengths of the current
+    // solve (smooth_lengths), chosen from them by choose_lengths
+    bool wide_rho = false, wide_cotangents = false, smooth = false;
     Workspace ws;
     DepositBins bins;
     void *efi = nullptr;  // node-interleaved field for the interpolation gather
@@ -250,12 +256,14 @@ struct Mesh {
     int slice_log2 = kSliceLog2Default;
 };
 
-// Remembers the widest particles deposited on a Float32 mesh (the lengths of
-// its transforms, smooth_lengths).
-inline void note_particles(Mesh *m, int pdt)
+// Remembers the type of the particles deposited into rho, n of them.
+inline void note_charges(Mesh *m, int pdt, int64_t n, int clear)
 {
-    if (pdt == SC_F64 && m->dtype == SC_F32) m->f64_particles = true;
+    m->wide_rho = (m->wide_rho && !clear) || (n > 0 && pdt == SC_F64 && m->dtype == SC_F32);
 }
+
+// Chooses the transform lengths (smooth_lengths) of the mesh's next solve.
+void choose_lengths(Mesh *m, bool adjoint);
 
 constexpr int kChunkLog2Min = 10, kChunkLog2Max = 14;
 constexpr int kSliceLog2Min = 10, kSliceLog2Max = 13;

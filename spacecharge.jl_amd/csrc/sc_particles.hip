@@ -728,7 +728,6 @@ int launch_deposit_to(Mesh *m, int pdt, const void *x, const void *y, const void
     const int rc = launch_deposit_binned(m, pdt, x, y, z, q, n, lo, dl, clear, out);
     if (rc != SC_ERR_UNSUPPORTED) return rc;
     // more tiles than the binned path holds: one atomic per node contribution
-    note_particles(m, pdt);
     if (clear) {
         if (int rc2 = launch_clear(m->ctx, out, rho_bytes)) return rc2;
     }
@@ -750,6 +749,7 @@ int launch_deposit(Mesh *m, int pdt, const void *x, const void *y, const void *z
     // marks where this deposit starts on the stream; a following solve's
     // Green build (side stream) waits for it, see run_solve
     if (int rc = mark_deposit_start(m)) return rc;
+    note_charges(m, pdt, n, clear);
     return launch_deposit_to(m, pdt, x, y, z, q, n, lo, dl, clear, m->rho);
 }
 
@@ -848,6 +848,7 @@ int launch_interp_vjp(Mesh *m, int pdt, const void *x, const void *y, const void
         // Its start is a deposit start: a following (adjoint) solve's Green
         // build forks there and runs beside it
         if (int rc = mark_deposit_start(m)) return rc;
+        m->wide_cotangents = n > 0 && pdt == SC_F64 && m->dtype == SC_F32;
         const void *gE[3] = {gEx, gEy, gEz};
         void *outs[3];
         for (int c = 0; c < 3; ++c) outs[c] = static_cast<char *>(g_efield) + (size_t)c * M * m->dtype;

@@ -371,7 +371,7 @@ int run_solve(Mesh *m, const double lo[3], const double hi[3], const double dl[3
     // the Green kernels read it there; the host cannot key a cache on it
     const bool devgeom = dl == nullptr;
     const double offz = devgeom ? 0.0 : lo[2] + hi[2];  // 2*zmin + (zmax - zmin), free_space.jl:39
-    double key[6] = {0.0, 0.0, 0.0, gamma, 0.0, (double)gmode};
+    double key[7] = {0.0, 0.0, 0.0, gamma, 0.0, (double)gmode, m->smooth ? 1.0 : 0.0};
     if (!devgeom) {
         for (int a = 0; a < 3; ++a) key[a] = dl[a];
         key[4] = cath ? offz : 0.0;
@@ -532,9 +532,10 @@ int run_solve(Mesh *m, const double lo[3], const double hi[3], const double dl[3
 int run_solve_io(Mesh *m, const double lo[3], const double hi[3], const double dl[3], double gamma,
                  SolveIO io)
 {
+    const bool adj = mode_adjoint(io.mode);
+    choose_lengths(m, adj);
     int rc = ensure_workspace(m);
     if (rc != SC_OK) return rc;
-    const bool adj = mode_adjoint(io.mode);
     io.fwd = adj ? m->ws.B : m->ws.A;
     io.inv = adj ? m->ws.A : m->ws.B;
     if (m->dtype == SC_F32) return run_solve<float>(m, lo, hi, dl, gamma, io);
@@ -613,45 +614,76 @@ void free_workspace(Mesh *m)
     if (m->ctx && m->ctx->side) (void)hipStreamSynchronize(m->ctx->side);
     if (ws.green_done) (void)hipEventDestroy(ws.green_done);
     if (ws.deposit_start) (void)hipEventDestroy(ws.deposit_start);
-    void *ptrs[] = {ws.A, ws.B, ws.Gf, ws.Gi, ws.F, ws.R, ws.twT[0], ws.twT[1], ws.twT[2]};
+    void *ptrs[] = {ws.A, ws.B, ws.Gf, ws.Gi, ws.F, ws.R};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
+    for (int a = 0; a < 3; ++a) {
+        if (ws.twSet[0][a]) (void)hipFree(ws.twSet[0][a]);
+        if (ws.twSet[1][a] && ws.twSet[1][a] != ws.twSet[0][a]) (void)hipFree(ws.twSet[1][a]);
+    }
     ws = Workspace();
+}
+
+void choose_lengths(Mesh *m, bool adjoint)
+{
+    m->smooth = m->dtype == SC_F32 && (adjoint ? m->wide_cotangents : m->wide_rho);
 }
 
 int ensure_workspace(Mesh *m)
 {
     Workspace &ws = m->ws;
-    if (ws.ready) return SC_OK;
+    auto take_lengths = [&]() {
+        for (int a = 0; a < 3; ++a) {
+            ws.twT[a] = ws.twSet[m->smooth][a];
+            ws.plan[a] = ws.planSet[m->smooth][a];
+        }
+    };
+    if (ws.ready) {
+        take_lengths();
+        return SC_OK;
+    }
     Ctx *ctx = m->ctx;
-    const Dims d = make_dims(m);
-    ws.smooth = smooth_lengths(m);
-    // transform half-lengths (padded beyond the mesh's nodes, see transform_half)
-    const int64_t nx = d.nx, ny = d.ny, nz = d.nz;
-    const int L[3] = {d.Lx, d.Ly, d.Lz};
-    const int64_t mn[3] = {m->n[0], m->n[1], m->n[2]};
+    // both sets of lengths of a Float32 mesh: a later solve may be under capture
+    const int sets = m->dtype == SC_F32 ? 2 : 1;
+    const bool smooth = m->smooth;
+    Dims dims[2];
+    for (int k = 0; k < sets; ++k) {
+        m->smooth = k == 1;
+        dims[k] = make_dims(m);
+    }
+    m->smooth = smooth;
     const int cap = (m->dtype == SC_F32) ? fft_cap_xl<float>() : fft_cap_xl<double>();
-    for (int a = 0; a < 3; ++a) {
-        // one pencil must fit one workgroup (registers and LDS)
-        if (L[a] > cap)
-            return set_err(ctx, SC_ERR_UNSUPPORTED,
-                           "grid size " + std::to_string(mn[a]) + " needs a transform of length " +
-                               std::to_string(L[a]) + ", beyond the maximum of " +
-                               std::to_string(cap) + " for this mesh type (at most " +
-                               std::to_string(cap / 2) + " nodes per axis)");
-        if (!make_plan(L[a], &ws.plan[a]))  // unreachable: transform_half gives 7-smooth lengths
-            return set_err(ctx, SC_ERR_UNSUPPORTED,
-                           "no transform plan for length " + std::to_string(L[a]));
+    for (int k = 0; k < sets; ++k) {
+        // transform half-lengths (padded beyond the mesh's nodes, see transform_half)
+        const int L[3] = {dims[k].Lx, dims[k].Ly, dims[k].Lz};
+        for (int a = 0; a < 3; ++a) {
+            // one pencil must fit one workgroup (registers and LDS)
+            if (L[a] > cap)
+                return set_err(ctx, SC_ERR_UNSUPPORTED,
+                               "grid size " + std::to_string(m->n[a]) + " needs a transform of length " +
+                                   std::to_string(L[a]) + ", beyond the maximum of " +
+                                   std::to_string(cap) + " for this mesh type (at most " +
+                                   std::to_string(cap / 2) + " nodes per axis)");
+            if (!make_plan(L[a], &ws.planSet[k][a]))  // unreachable: transform_half gives 7-smooth lengths
+                return set_err(ctx, SC_ERR_UNSUPPORTED,
+                               "no transform plan for length " + std::to_string(L[a]));
+        }
     }
     const size_t s = (m->dtype == SC_F32) ? 4 : 8;
-    const size_t Kp = d.Kp;  // row stride of every kx-indexed array
-    // complex elements of one spectrum: [mesh z][Ly][Kp]
-    const size_t spec = (size_t)d.mz * d.Ly * Kp;
-    const size_t gf = (size_t)(nz + 1) * (ny + 1) * Kp;
-    const size_t gi = (size_t)2 * nz * (ny + 1) * Kp;
-    // Green build scratch: F at the nodes (Float64), R rows (T), free + image
-    const size_t fn = (size_t)(nx + 1) * (ny + 1) * ((nz + 1) + 2 * nz);
-    const size_t rn = (size_t)(ny + 1) * Kp * (nz + (2 * nz - 1));
+    size_t spec = 0, gf = 0, gi = 0, fn = 0, rn = 0;  // of the longer set
+    auto most = [](size_t &a, size_t b) { a = b > a ? b : a; };
+    for (int k = 0; k < sets; ++k) {
+        const Dims &d = dims[k];
+        const int64_t nx = d.nx, ny = d.ny, nz = d.nz;
+        const size_t Kp = d.Kp;  // row stride of every kx-indexed array
+        // complex elements of one spectrum: [mesh z][Ly][Kp]
+        most(spec, (size_t)d.mz * d.Ly * Kp);
+        most(gf, (size_t)(nz + 1) * (ny + 1) * Kp);
+        most(gi, (size_t)2 * nz * (ny + 1) * Kp);
+        // Green build scratch: F at the nodes (Float64), R rows (T), free + image
+        most(fn, (size_t)(nx + 1) * (ny + 1) * ((nz + 1) + 2 * nz));
+        most(rn, (size_t)(ny + 1) * Kp * (nz + (2 * nz - 1)));
+    }
     auto fail = [&](void) {
         free_workspace(m);
         return set_err(ctx, SC_ERR_NOMEM, "device allocation of the solver workspace failed");
@@ -663,13 +695,21 @@ int ensure_workspace(Mesh *m)
     if (hipMalloc((void **)&ws.F, sizeof(double) * 3 * fn) != hipSuccess) return fail();
     if (hipMalloc(&ws.R, s * 3 * rn) != hipSuccess) return fail();
     ws.bytes = (int64_t)(8 * s * spec + 3 * s * gf + 6 * s * gi + 24 * fn + 3 * s * rn);
-    for (int a = 0; a < 3; ++a) {
-        int rc = (m->dtype == SC_F32) ? upload_twiddles<float>(ctx, L[a], &ws.twT[a])
-                                      : upload_twiddles<double>(ctx, L[a], &ws.twT[a]);
-        if (rc != SC_OK) { free_workspace(m); return rc; }
+    for (int k = 0; k < sets; ++k) {
+        const int L[3] = {dims[k].Lx, dims[k].Ly, dims[k].Lz}, L0[3] = {dims[0].Lx, dims[0].Ly, dims[0].Lz};
+        for (int a = 0; a < 3; ++a) {
+            if (k > 0 && L[a] == L0[a]) {
+                ws.twSet[k][a] = ws.twSet[0][a];
+                continue;
+            }
+            int rc = (m->dtype == SC_F32) ? upload_twiddles<float>(ctx, L[a], &ws.twSet[k][a])
+                                          : upload_twiddles<double>(ctx, L[a], &ws.twSet[k][a]);
+            if (rc != SC_OK) { free_workspace(m); return rc; }
+        }
     }
     ws.dtype = m->dtype;
     ws.ready = true;
+    take_lengths();
     return SC_OK;
 }
 
@@ -696,8 +736,8 @@ int solve_adjoint_mesh(Mesh *m, const double lo[3], const double hi[3], const do
 
 
 // ---- grouped solves: same-shape bunches of a batched solve ----
-// The bunches of one class (mesh shape, type, cathode flag; register-engine
-// lengths) run each Green and transform kernel once for all of them, with
+// The bunches of one class (mesh shape, type, cathode flag and lengths, all
+// register-engine ones) run each Green and transform kernel once for all of them, with
 // their buffers and Green geometry from a table in the context's device
 // memory, written by store launches that carry the entries as arguments
 // (so a captured graph rewrites them on every replay).  Each class owns a
@@ -727,8 +767,10 @@ int solve_class_t(Ctx *ctx, Mesh *const *ms, int k, const double *const *lo, con
 {
     hipStream_t st = ctx->stream;
     const int mode = cath ? kFieldCathode : kFieldFree;
-    for (int i = 0; i < k; ++i)
+    for (int i = 0; i < k; ++i) {
+        choose_lengths(ms[i], false);
         if (int rc = ensure_workspace(ms[i])) return rc;
+    }
     const Dims d = make_dims(ms[0]);
     const double P = (double)d.Lx * (double)d.Ly * (double)d.Lz;
     SStore s;

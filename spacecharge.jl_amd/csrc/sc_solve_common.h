@@ -87,16 +87,14 @@ inline bool padding_pays(const Mesh *m)
     return r <= (far ? 1.2 : 4.0 / 3.0);
 }
 
-// Float32 meshes that carry Float64 particles keep the plain 7-smooth lengths
-// (and with them the generic engine, except for unpadded powers of two).
-// Their caller gets the interpolated fields in Float64 and so sees the
-// transforms' Float32 rounding itself, which any other length or radix moves
-// by 1e-7 of the field: such fields stay reproducible to the last bits.  The
-// choice is made when the mesh's workspace is, by the particles deposited so far.
-inline bool smooth_lengths(const Mesh *m)
-{
-    return m->ws.ready ? m->ws.smooth : m->f64_particles && m->dtype == SC_F32;
-}
+// Solves of a Float32 mesh whose rho was deposited from Float64 particles (adjoint
+// solves: whose cotangents were) keep the plain 7-smooth lengths, and with them the
+// generic engine, except for unpadded powers of two.  Their caller gets the
+// interpolated fields in Float64 and so sees the transforms' Float32 rounding
+// itself, which any other length or radix moves by 1e-7 of the field: such fields
+// are the same bits whatever ran on the mesh before.  The choice is that of the
+// solve alone (choose_lengths); the workspace holds both sets of lengths.
+inline bool smooth_lengths(const Mesh *m) { return m->smooth; }
 
 // Shape of a solve.  nx, ny, nz are the transform half-lengths (the Green
 // function's lags and spectral octant); mx, my, mz the mesh's nodes (the
@@ -147,7 +145,7 @@ inline Engine engine_of(const Mesh *m, int L, bool padded)
 // 32^3 36.7 / 31.1, 32x32x512 164 / 155, 50^3 47.6 / 41.9, 64^3 60.9 / 56.0, 64x64x256
 // 129 / 121, 65x65x129 90.4 / 90.0; Float64 16^3 30.6 / 26.4, 32^3 36.1 / 32.2,
 // 32x32x512 234 / 220, 50^3 56.1 / 52.8, 48x48x96 73.2 / 73.1, 48x48x256 122 / 116; and
-// two launches fewer for the host.  Meshes with smooth_lengths keep their bits, and
+// two launches fewer for the host.  Solves with smooth_lengths keep their bits, and
 // force_generic_transforms its engine.
 inline bool plane_lengths(const Mesh *m, const Dims &d)
 {
