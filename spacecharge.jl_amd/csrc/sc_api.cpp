@@ -927,6 +927,7 @@ int sc_solve_batched(sc_mesh *const *meshes, int nb, const double *min_bounds,
             return set_err(c, SC_ERR_INVALID, "max_bounds must be finite");
     }
     if (int e = check_dev(c)) return e;
+    for (int b = 0; b < nb; ++b) choose_lengths(&meshes[b]->m, false);
     int table = SC_ERR_UNSUPPORTED;
     if ((c->grouped & SC_GROUP_SOLVE) && nb > 1) {
         table = ensure_solve_table(c);  // SC_ERR_UNSUPPORTED: first needed under capture
@@ -952,6 +953,7 @@ int sc_solve_batched(sc_mesh *const *meshes, int nb, const double *min_bounds,
                     const Mesh &mo = meshes[o]->m;
                     if (!done[o] && solve_groupable(&mo) && mo.dtype == mb.dtype &&
                         mo.n[0] == mb.n[0] && mo.n[1] == mb.n[1] && mo.n[2] == mb.n[2] &&
+                        mo.smooth == mb.smooth &&
                         (at_cathode[o] != 0) == (at_cathode[b] != 0)) {
                         cls.push_back(o);
                         done[o] = true;

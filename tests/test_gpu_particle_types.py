@@ -81,6 +81,28 @@ def test_adjoint_does_not_depend_on_earlier_particle_types(grid):
             assert torch.equal(grad(mesh, q), want[q[0].dtype])
 
 
+@pytest.mark.parametrize("order", [(0, 1, 0, 1), (1, 0, 1, 0)])
+@pytest.mark.parametrize("grid", [(32, 32, 32), (16, 16, 16), (20, 33, 26)])
+def test_batch_of_both_kinds_equals_single_solves(grid, order):
+    import spacecharge as sc
+    parts = [_bunch((torch.float32, torch.float64)[k], 20 + i) for i, k in enumerate(order)]
+    want = []
+    for p in parts:
+        m = _mesh(grid)
+        sc.deposit(m, *p)
+        sc.solve(m)
+        want.append(m.efield.clone())
+    meshes = [_mesh(grid) for _ in parts]
+    for rep in range(2):
+        for m, p in zip(meshes, parts):
+            sc.deposit(m, *p)
+        sc.solve_batched(meshes)
+        torch.cuda.synchronize()
+        for m, w in zip(meshes, want):
+            assert torch.equal(m.efield, w)
+            m.efield.zero_()
+
+
 def test_captured_step_of_either_kind_after_one_of_the_other():
     """One eager step of either kind prepares the capture of the other."""
     grid = (20, 33, 26)
