@@ -1081,10 +1081,19 @@ k_green_3m(const T *__restrict__ R, T *__restrict__ Gf, cpx<T> *__restrict__ Gi,
 // (differences along x, then z, then y, as diff8v) of S rows, which go through
 // the x transform in place.  The node rows that neighbouring workgroups share
 // are evaluated twice (1/S more, and 1/K more along z for K planes).
-// The values are k_green_f3's: the same terms in the same order; the column
-// and row logs of a plane come from LDS tables, as does log(u^2 + v^2) of each
-// node (one node at a time per lane: with a lane's nodes unrolled the kernel
+// The terms and their order are k_green_f3's; the column and row logs of a plane
+// come from LDS tables, as does log(u^2 + v^2) of each node (one node at a time per lane: with a lane's nodes unrolled the kernel
 // took 238 VGPRs instead of 192 at 256 points and the 128^3 build 79 us, not 75).
+// Squares and their sums are rounded one by one: with the compiler's choice of
+// fused forms, which differed between r and the tables, the field of a Float64
+// mesh lay 4-5% further from a plain 64-bit evaluation than with k_green_f3
+// (32^3 1.08e-14 against 1.02e-14; from extended precision both 6.9e-14).
+__device__ __forceinline__ double sum_squares(double a, double b, double c = 0.0)
+{
+#pragma clang fp contract(off)
+    return (a * a + b * b) + c * c;
+}
+
 template <typename T, int L>
 struct FxShape {
     static constexpr int E = Shape<T, L>::E, TPP = Shape<T, L>::TPP;
@@ -1130,10 +1139,10 @@ k_green_fx(T *__restrict__ R, const cpx<T> *__restrict__ twg, GreenArgs a, int s
         return image ? ((double)(k - a.d.nz) + 0.5) * dz + offzg : ((double)k - 0.5) * dz;
     };
     auto tables = [&](int k) {
-        const double w = coord_w(k), ww = w * w;
+        const double w = coord_w(k);
         for (int t = threadIdx.x; t < X::ROWS + NXN; t += TH) {
             const double s = t < NXN ? coord_u(t) : coord_v(y0 + t - NXN);
-            const double q = log_<FAST>(ww + s * s);
+            const double q = log_<FAST>(sum_squares(s, w));
             if (t < NXN) qwu_t[k & 1][t] = q;
             else qvw_t[k & 1][t - NXN] = q;
         }
@@ -1141,7 +1150,7 @@ k_green_fx(T *__restrict__ R, const cpx<T> *__restrict__ twg, GreenArgs a, int s
     // read back by the lane that writes it
     for (int n = threadIdx.x; n < X::NODES; n += TH) {
         const double u = coord_u(n % NXN), v = coord_v(y0 + n / NXN);
-        Quv[n] = log_<FAST>(u * u + v * v);
+        Quv[n] = log_<FAST>(sum_squares(u, v));
     }
     tables(k0);
     // this lane's pencil: component c, rows y0 + 2 pair and the next
@@ -1155,14 +1164,13 @@ k_green_fx(T *__restrict__ R, const cpx<T> *__restrict__ twg, GreenArgs a, int s
     double prev[3][E / 2];
     __syncthreads();
     for (int kn = k0; kn <= k1; ++kn) {
-        const double w = coord_w(kn), ww = w * w;
+        const double w = coord_w(kn);
 #pragma unroll 1
         for (int n = threadIdx.x; n < X::NODES; n += TH) {
             {
                 const int i = n % NXN, rw = n / NXN;
                 const double u = coord_u(i), v = coord_v(y0 + rw);
-                const double uu = u * u, vv = v * v;
-                const double r = sqrt((uu + vv) + ww);
+                const double r = sqrt(sum_squares(u, v, w));
                 const double Lu = log_<FAST>(r + u), Lv = log_<FAST>(r + v), Lw = log_<FAST>(r + w);
                 const double ax = atan_q<FAST>(v * w, r * u);
                 const double ay = atan_q<FAST>(w * u, r * v);
