@@ -155,7 +155,6 @@ __device__ __forceinline__ void dft(cpx<T> *v)
     else if constexpr (R == 12) dft_pf<4, 3, DIR>(v);
     else if constexpr (R == 16) reg::dft16<DIR>(v);
     else if constexpr (R == 20) dft_pf<4, 5, DIR>(v);
-    else if constexpr (R == 24) dft_pf<8, 3, DIR>(v);
     else static_assert(R == 2, "no butterfly of this radix");
 }
 

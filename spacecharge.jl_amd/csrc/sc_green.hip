@@ -1102,7 +1102,6 @@ struct FxShape {
     static constexpr int FFT = NP * TPP;                // lanes of the transforms
     static constexpr int THREADS = FFT <= 256 ? 256 : FFT;
     static constexpr int NXN = L / 2 + 1, ROWS = S + 1, NODES = ROWS * NXN;
-    static constexpr int M = (NODES + THREADS - 1) / THREADS;  // nodes per lane
     static constexpr int SLICE = reg::padded<L, E>();
     static constexpr size_t F_BYTES = sizeof(double) * 3 * NODES;
     static constexpr size_t T_BYTES = sizeof(cpx<T>) * (NP + 1) * SLICE;  // one slice for idle lanes

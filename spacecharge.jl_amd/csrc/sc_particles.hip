@@ -220,11 +220,10 @@ __device__ __forceinline__ void interp_body(
 }
 
 // Float64 fields: at most 4 waves per SIMD, so that the compiler may keep
-// every gather of a particle in flight at once (70 VGPRs).  Left to its own
-// occupancy target it fitted 62 VGPRs by issuing the z components' loads
-// only after the first loads had returned, a second memory round trip: on
-// 4M particles, 128^3, the gather went from 240 to 210 us (node pairs) and
-// from 303 to 264 us (one node per entry).
+// every gather of a particle in flight at once.  Left to its own occupancy
+// target it issues some loads only after the first have returned, a second
+// memory round trip (copy and gather, us, without / with: 4M particles on 128^3
+// packed 206 / 176, padded 233 / 216; 2M on 64x64x128 78 / 67; 8M on 256^3 784 / 777).
 template <typename PT, typename MT, int PP>
 __global__ void __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(1, sizeof(MT) == 8 ? 4 : 8)))
@@ -232,10 +231,10 @@ k_interp(const typename V4<MT>::type *__restrict__ efi, const PT *__restrict__ p
          const PT *__restrict__ py, const PT *__restrict__ pz, int64_t n, int nx, int ny, int nz,
          double lx_, double ly_, double lz_, double dx_, double dy_, double dz_,
          const double *__restrict__ geom, PT *__restrict__ Ex, PT *__restrict__ Ey,
-         PT *__restrict__ Ez, int P)
+         PT *__restrict__ Ez)
 {
     interp_body<PT, MT, PP>((int64_t)blockIdx.x * blockDim.x + threadIdx.x, efi, px, py, pz, n, nx,
-                            ny, nz, lx_, ly_, lz_, dx_, dy_, dz_, geom, Ex, Ey, Ez, P);
+                            ny, nz, lx_, ly_, lz_, dx_, dy_, dz_, geom, Ex, Ey, Ez, PP);
 }
 
 // The gather straight from the three component arrays, without the interleaved
@@ -390,7 +389,7 @@ k_deposit_vjp(const MT *__restrict__ g, const PT *__restrict__ px, const PT *__r
 
 // Position part of the VJP of interpolation at cotangents (gEx, gEy, gEz):
 // g_pos = sum_c gE_c * d/dpos (sum_8 w E_c), from the interleaved field
-// (entry layout PP, as P).
+// (entry layout PP).
 template <typename PT, typename MT, int PP>
 __global__ void __launch_bounds__(256)
 k_interp_vjp(const typename V4<MT>::type *__restrict__ efi, const PT *__restrict__ px,
@@ -398,7 +397,7 @@ k_interp_vjp(const typename V4<MT>::type *__restrict__ efi, const PT *__restrict
              const PT *__restrict__ gEy, const PT *__restrict__ gEz, int64_t n, int nx, int ny,
              int nz, double lx_, double ly_, double lz_, double dx_, double dy_, double dz_,
              const double *__restrict__ geom, PT *__restrict__ gx, PT *__restrict__ gy,
-             PT *__restrict__ gz, int accumulate, int P)
+             PT *__restrict__ gz, int accumulate)
 {
 #pragma clang fp contract(off)
     using C = wider_t<PT, MT>;
@@ -622,7 +621,7 @@ void itp(Mesh *m, const void *efi, int P, const void *x, const void *y, const vo
                        m->ctx->stream, static_cast<const typename V4<MT>::type *>(efi),
                        (const PT *)x, (const PT *)y, (const PT *)z, n, (int)m->n[0], (int)m->n[1],
                        (int)m->n[2], h.l[0], h.l[1], h.l[2], h.d[0], h.d[1], h.d[2], h.dev,
-                       (PT *)Ex, (PT *)Ey, (PT *)Ez, P);
+                       (PT *)Ex, (PT *)Ey, (PT *)Ez);
 }
 
 }  // namespace
@@ -654,7 +653,7 @@ void itp_vjp(Mesh *m, const void *x, const void *y, const void *z, int64_t n, co
                        (const PT *)x, (const PT *)y, (const PT *)z, (const PT *)gEx, (const PT *)gEy,
                        (const PT *)gEz, n, (int)m->n[0], (int)m->n[1], (int)m->n[2], h.l[0], h.l[1],
                        h.l[2], h.d[0], h.d[1], h.d[2], h.dev, (PT *)gx, (PT *)gy, (PT *)gz,
-                       accumulate, m->efi_pair);
+                       accumulate);
 }
 
 // Whether the interpolation of n particles gathers straight from efield: the
