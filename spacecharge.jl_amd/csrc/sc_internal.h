@@ -234,10 +234,12 @@ struct Mesh {
     bool owns = false;
     bool green_reuse = false;
     bool generic_transforms = false;  // diagnostic: skip the register-resident engine
-    // a Float32 mesh: Float64 particles went into rho since it was last cleared,
-    // or into the last cotangent deposit; smooth: the lengths of the current
-    // solve (smooth_lengths), chosen from them by choose_lengths
-    bool wide_rho = false, wide_cotangents = false, smooth = false;
+    // a Float32 mesh: Float64 particles went into rho since it was last cleared;
+    // the same of the last cotangent deposit (-1: none since the last charges);
+    // smooth: the lengths of the current solve (smooth_lengths), chosen from them
+    // by choose_lengths
+    bool wide_rho = false, smooth = false;
+    int wide_cotangents = -1;
     Workspace ws;
     DepositBins bins;
     void *efi = nullptr;  // node-interleaved field for the interpolation gather
@@ -260,6 +262,7 @@ struct Mesh {
 inline void note_charges(Mesh *m, int pdt, int64_t n, int clear)
 {
     m->wide_rho = (m->wide_rho && !clear) || (n > 0 && pdt == SC_F64 && m->dtype == SC_F32);
+    m->wide_cotangents = -1;
 }
 
 // Chooses the transform lengths (smooth_lengths) of the mesh's next solve.

@@ -626,7 +626,8 @@ void free_workspace(Mesh *m)
 
 void choose_lengths(Mesh *m, bool adjoint)
 {
-    m->smooth = m->dtype == SC_F32 && (adjoint ? m->wide_cotangents : m->wide_rho);
+    const bool cotangents = adjoint && m->wide_cotangents >= 0;
+    m->smooth = m->dtype == SC_F32 && (cotangents ? m->wide_cotangents > 0 : m->wide_rho);
 }
 
 int ensure_workspace(Mesh *m)

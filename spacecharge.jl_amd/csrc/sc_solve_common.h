@@ -88,7 +88,7 @@ inline bool padding_pays(const Mesh *m)
 }
 
 // Solves of a Float32 mesh whose rho was deposited from Float64 particles (adjoint
-// solves: whose cotangents were) keep the plain 7-smooth lengths, and with them the
+// solves: whose cotangents were, if any were since) keep the plain 7-smooth lengths, and with them the
 // generic engine, except for unpadded powers of two.  Their caller gets the
 // interpolated fields in Float64 and so sees the transforms' Float32 rounding
 // itself, which any other length or radix moves by 1e-7 of the field: such fields

@@ -81,6 +81,28 @@ def test_adjoint_does_not_depend_on_earlier_particle_types(grid):
             assert torch.equal(grad(mesh, q), want[q[0].dtype])
 
 
+@pytest.mark.parametrize("grid", GRIDS)
+def test_adjoint_of_given_cotangents_follows_the_charges(grid):
+    """Without a cotangent deposit the adjoint takes the field solve's lengths, and its
+    Green spectra where they are reused."""
+    import spacecharge as sc
+    narrow, wide = _bunch(torch.float32), _bunch(torch.float64, 6)
+    g = torch.rand((*grid, 3), generator=torch.Generator(device=DEV).manual_seed(1), device=DEV)
+    mesh = _mesh(grid)
+    mesh.set_green_reuse()
+    for p in (narrow, wide, narrow):
+        fresh = _mesh(grid)
+        sc.deposit(fresh, *p)
+        want = sc.solve_adjoint(fresh, g).clone()
+        sc.interpolate_adjoint(mesh, *wide[:3], *wide[1:4], positions=False)
+        sc.deposit(mesh, *p)
+        sc.solve(mesh)
+        with sc.KernelTimer() as t:
+            got = sc.solve_adjoint(mesh, g)
+        assert not any(k.startswith("green") for k in t.results())
+        assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("order", [(0, 1, 0, 1), (1, 0, 1, 0)])
 @pytest.mark.parametrize("grid", [(32, 32, 32), (16, 16, 16), (20, 33, 26)])
 def test_batch_of_both_kinds_equals_single_solves(grid, order):
