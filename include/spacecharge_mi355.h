@@ -107,9 +107,9 @@ int sc_mesh_force_generic_transforms(sc_mesh *mesh, int enable);
  * field copy that the interpolation and its adjoint gather from.  layout 1
  * holds one padded (Ex, Ey, Ez, 0) entry per node; layout 2 packs the three
  * values of a node, so that the node pairs of a cell along x are one run of six
- * (Float64 meshes only); 0 (the default) lets the library choose: packed for
- * Float64 meshes and for small and very large Float32 ones, and no copy at all
- * where the particles are few per node.
+ * (it can be asked for on Float64 meshes only); 0 (the default) lets the library
+ * choose: packed for Float64 meshes and for small and very large Float32 ones,
+ * and no copy at all for few particles (100,000; more on very large meshes).
  * Results are the same bits in every layout.  Changing it synchronises the
  * context's stream and frees the current copy. */
 int sc_mesh_set_field_layout(sc_mesh *mesh, int layout);
@@ -219,9 +219,9 @@ int sc_interpolate(sc_mesh *mesh, int pdtype, const void *x, const void *y, cons
 
 /* No counterpart in the reference: sc_interpolate for callers that cannot
  * allocate device memory (code under stream or graph capture, tight serving
- * loops, harnesses that forbid hipMalloc).  Same arguments, same kernels and
- * the same bits as sc_interpolate, but it calls no hipMalloc, hipFree or
- * allocating library routine: the node-interleaved field copy lives in a
+ * loops, harnesses that forbid hipMalloc).  Same arguments and the same bits
+ * as sc_interpolate, always by the padded field copy (layout 1), but it calls
+ * no hipMalloc, hipFree or allocating library routine: the copy lives in a
  * fixed 64 MiB array per GPU, held from library load until the process ends,
  * instead of the mesh's own buffer.  That limits the mesh to 4,194,304 nodes
  * (Float32, e.g. 160^3) or 2,097,152 nodes (Float64, e.g. 128^3); larger
@@ -303,16 +303,23 @@ int sc_interpolate_adjoint(sc_mesh *mesh, int pdtype, const void *x, const void 
  *    interpolation (2) as ONE launch over the workgroups of all bunches, on
  *    the context's stream;
  *  - SC_GROUP_SOLVE: sc_solve_batched solves each class of two or more
- *    meshes of one shape, type and cathode flag (transform lengths 32..512,
- *    no Green reuse, at most 64 MB of spectra per class, so small meshes)
- *    with one launch per Green and transform kernel; classes and the other
- *    bunches share the stream pool.
+ *    meshes of one shape, type and cathode flag (axes of up to 256 nodes, no
+ *    Green reuse, at most 64 MB of spectra per class, so small meshes; Float32
+ *    meshes with Float32 and with Float64 particles apart, and the latter only
+ *    with axes of 16 to 256 nodes that are powers of two) with one launch per
+ *    Green and transform kernel; classes and the other bunches share the
+ *    stream pool.
  * The per-bunch descriptors go to tables in the context's device memory
  * through store launches that carry them as kernel arguments, so a graph
  * capture replays them; grouped calls of one context must not overlap
  * (they share the tables).  The first grouped call allocates the tables and
  * must run outside stream capture (under capture it falls back to the pool).
- * Results are the same bits as the pool path for Float32 meshes. */
+ * Solves and interpolations give the same bits as the pool path for Float32
+ * meshes.  So does the deposit where both bin the particles.  Bunches that a
+ * single deposit takes without binning (few particles on small meshes) are added
+ * up in another grouping: the same contributions in Float64 sums that agree to a
+ * few 1e-16, so the same Float32 values but for the rare sum (about one node in
+ * 1e8) that lies that close to a rounding boundary. */
 #define SC_GROUP_PARTICLES 1
 #define SC_GROUP_SOLVE 2
 int sc_ctx_set_pool_size(sc_ctx *ctx, int nstreams);

@@ -818,8 +818,10 @@ k_gather_tiles(const double *__restrict__ partials, size_t pstride,
 //
 // Float32 meshes accumulate in fixed point by the binned chain's rules (the
 // scale from max|q| over all particles, Float64 in tiles that hold a particle
-// with weights outside [0, 1]), so that both give the same bits; a launch
-// before it (k_direct_prep) finds the two.
+// with weights outside [0, 1]); a launch before it (k_direct_prep) finds the
+// two.  Both paths so add the same contributions, exactly within a sub-grid;
+// the sub-grids hold other particles, and their Float64 sums agree to a few
+// 1e-16: the same Float32 values unless that straddles a rounding boundary.
 
 // max|q| of each channel and the mask of tiles that hold an extrapolating
 // particle, per slice of the particles (workgroup w: qmax[c * kBinMaxSlices +

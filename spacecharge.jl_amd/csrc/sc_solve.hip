@@ -693,6 +693,8 @@ int ensure_workspace(Mesh *m)
     if (hipMalloc(&ws.B, 3 * 2 * s * spec) != hipSuccess) return fail();
     if (hipMalloc(&ws.Gf, 3 * s * gf) != hipSuccess) return fail();
     if (hipMalloc(&ws.Gi, 3 * 2 * s * gi) != hipSuccess) return fail();
+    // (F also where every field solve takes the fused Green kernel, which does not
+    // store it: a potential solve does, and may come under capture)
     if (hipMalloc((void **)&ws.F, sizeof(double) * 3 * fn) != hipSuccess) return fail();
     if (hipMalloc(&ws.R, s * 3 * rn) != hipSuccess) return fail();
     ws.bytes = (int64_t)(8 * s * spec + 3 * s * gf + 6 * s * gi + 24 * fn + 3 * s * rn);

@@ -298,7 +298,7 @@ class Mesh3D:
         copy: 1 = one padded entry per node, 2 = packed, so that the node pairs
         along x are one run (Float64 meshes only), 0 = picked by the library
         (packed for Float64 meshes and for small and very large Float32 ones,
-        and no copy at all for few particles per node)."""
+        and no copy at all for few particles)."""
         ctx = _ctx(self.device)
         with _on(self.device):
             rc = _lib.load().sc_mesh_set_field_layout(self._h, int(layout))
