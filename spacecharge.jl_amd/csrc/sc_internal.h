@@ -193,9 +193,9 @@ struct Workspace {
     // recorded after the z convolution of the last solve, where led < 2;
     // fork_capture: the id of the capture whose deposit recorded the event,
     // likewise (0: none).  A build with no usable record forks from the end of
-    // the stream.  captured: a capture has solved on this mesh; its replays,
-    // which may come between an eager deposit and its solve, clear no mark, so
-    // eager builds then always fork from the end.
+    // the stream.  captured: a capture has solved on this mesh or computed its
+    // bounds; its replays, which may come between an eager deposit and its
+    // solve, clear no mark, so eager builds then always fork from the end.
     // deposited: a deposit since the last solve; led: solves behind a deposit
     // since the last solve without one (2: two or more).
     hipEvent_t deposit_start = nullptr;

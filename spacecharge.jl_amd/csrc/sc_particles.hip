@@ -660,7 +660,7 @@ void itp_vjp(Mesh *m, const void *x, const void *y, const void *z, int64_t n, co
 // interleaved copy costs a launch and a pass over all M nodes, the direct gather
 // two to three times the cache lines per particle.  Particles spread over the
 // whole mesh miss most, so the line lies where these break even; those of a core
-// (rms a tenth of the mesh) would gain to twice the count.  Up to 200^3 nodes they
+// (rms a tenth of the mesh) would gain to twice the count.  Up to 160^3 nodes they
 // break even at about 100k particles whatever the mesh, beyond that the copy's
 // pass grows.  Measured, uniform particles, direct / copy (us), Float32: 100k on
 // 32^3 7.0 / 7.1, on 64^3 7.7 / 11.8, on 128^3 20.5 / 20.0 (core 8.9 / 16.1), 200k
@@ -923,6 +923,8 @@ int launch_bounds_geom(Mesh *m, int pdt, const void *x, const void *y, const voi
     }
     // a Green build that forked at an earlier deposit would read the geometry
     // while it is written
+    unsigned long long cid = 0;
+    if (stream_capturing(ctx->stream, &cid)) m->ws.captured = true;
     m->ws.fork_ready = false;
     m->ws.fork_capture = 0;
     int64_t nblk = 0;

@@ -401,8 +401,9 @@ int run_solve(Mesh *m, const double lo[3], const double hi[3], const double dl[3
             // the last z convolution that reads this mesh's Green spectra, and
             // after the bounds: an event of its own after each convolution, for
             // builds that fork further back, cost 5.5 us of idle device and 3 us
-            // of host time per solve.  A replayed graph leaves no trace here, so
-            // a mesh that a capture has solved on forks its eager builds at the end
+            // of host time per solve.  A replayed graph leaves no trace here, so a
+            // mesh that a capture has solved on, or computed the bounds of, forks
+            // its eager builds at the end
             const bool from_deposit = cap ? ws.fork_capture == cid : ws.fork_ready && !ws.captured;
             if (!from_deposit) SC_HIP(ctx, hipEventRecord(ws.deposit_start, st));
             SC_HIP(ctx, hipStreamWaitEvent(ctx->side, ws.deposit_start, 0));
@@ -489,7 +490,7 @@ int run_solve(Mesh *m, const double lo[3], const double hi[3], const double dl[3
     // a later build without a new deposit forks after this point: where the
     // stream ends then, or, on a mesh that was just solved without one, here,
     // so that it runs beside the backward passes (a loop of solves, 128^3
-    // Float32 207 -> 192 us each; deposit, field and potential 361 -> 340)
+    // Float32 207 -> 196 us each; deposit, field and potential 359 -> 337)
     ws.fork_capture = 0;
     ws.fork_ready = overlap && ws.led < 2 && !cap && !ws.captured;
     if (ws.fork_ready) SC_HIP(ctx, hipEventRecord(ws.deposit_start, st));

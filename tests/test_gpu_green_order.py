@@ -148,3 +148,32 @@ def test_replay_between_deposit_and_solve(T, batched):
         torch.cuda.synchronize()
         assert torch.equal(out, want[0]), rep
         assert torch.equal(got, want[1]), rep
+
+
+@pytest.mark.parametrize("T", [torch.float32, torch.float64])
+def test_replayed_bounds_between_deposit_and_solve(T):
+    """The same with bounds that a graph computes."""
+    sc, mesh, p = _setup(T)
+    live = [a.clone() for a in p[:3]]
+    mesh.update_bounds(*live)
+    sc.deposit(mesh, *p)
+    _run(sc, mesh, "field", 2.0)
+    torch.cuda.synchronize()
+    rho = mesh.rho.clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        mesh.update_bounds(*live)
+    for rep in range(4):
+        for a, b in zip(live, p):
+            a.copy_(b * (1.0 + 0.25 * rep))
+        _, alone, _ = _setup(T)
+        alone.update_bounds(*live)
+        alone.rho.copy_(rho)
+        want = _run(sc, alone, "field", 2.0)
+        torch.cuda.synchronize()
+        sc.deposit(mesh, *p)
+        graph.replay()
+        mesh.rho.copy_(rho)
+        got = _run(sc, mesh, "field", 2.0)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want), rep
