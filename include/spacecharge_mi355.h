@@ -109,7 +109,8 @@ int sc_mesh_force_generic_transforms(sc_mesh *mesh, int enable);
  * values of a node, so that the node pairs of a cell along x are one run of six
  * (it can be asked for on Float64 meshes only); 0 (the default) lets the library
  * choose: packed for Float64 meshes and for small and very large Float32 ones,
- * and no copy at all for few particles (100,000; more on very large meshes).
+ * and no copy at all for few particles (125,000 in Float32, 160,000 in Float64,
+ * more on large meshes).
  * Results are the same bits in every layout.  Changing it synchronises the
  * context's stream and frees the current copy. */
 int sc_mesh_set_field_layout(sc_mesh *mesh, int layout);

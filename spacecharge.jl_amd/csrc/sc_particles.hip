@@ -658,22 +658,28 @@ void itp_vjp(Mesh *m, const void *x, const void *y, const void *z, int64_t n, co
 
 // Whether the interpolation of n particles gathers straight from efield: the
 // interleaved copy costs a launch and a pass over all M nodes, the direct gather
-// two to three times the cache lines per particle.  Particles spread over the
-// whole mesh miss most, so the line lies where these break even; those of a core
-// (rms a tenth of the mesh) would gain to twice the count.  Up to 160^3 nodes they
-// break even at about 100k particles whatever the mesh, beyond that the copy's
-// pass grows.  Measured, uniform particles, direct / copy (us), Float32: 100k on
-// 32^3 7.0 / 7.1, on 64^3 7.7 / 11.8, on 128^3 20.5 / 20.0 (core 8.9 / 16.1), 200k
-// on 128^3 39.8 / 29.1; 167k on 200^3 39 / 40, 350k on 256^3 82 / 97, 524k 122 / 106.
-// Float64: 100k on 32^3 7.7 / 8.7, on 64^3 12.7 / 17.6, on 100^3 20.9 / 21.0, 262k
-// on 128^3 58 / 42; 171k on 160^3 41 / 44, 333k on 200^3 83 / 103, 699k on 256^3
-// 171 / 212, 1.05M 255 / 244.  A forced layout keeps its copy.
+// two to three times the cache lines per particle, most of them missing where the
+// particles fill the mesh, few where they crowd in its core (rms a tenth of the
+// mesh, as bunches do).  The host cannot know which, so the line lies where a core
+// gains, in a whole step, about what uniform particles lose.  Steps with the
+// direct gather / the copy (us), core and uniform: Float32 131k on 64^3 99 / 103
+// and 98 / 103, 166k on 100^3 164 / 165 and 172 / 166, 131k on 128^3 241 / 253 and
+// 259 / 260, 200k 249 / 256 and 274 / 265, 349k 258 / 260 and 299 / 275, 682k on
+// 160^3 505 / 500 and 595 / 532, 524k on 256^3 1975 / 1998 and 2048 / 2040.
+// Float64: 131k on 64^3 113 / 117 and 110 / 113, 199k 120 / 120 and 121 / 117, 200k
+// on 100^3 226 / 232 and 247 / 238, 262k on 128^3 373 / 388 and 402 / 397, 349k 384 /
+// 396 and 424 / 406, 256k on 160^3 955 / 980 and 987 / 993.  The two calls alone
+// (replayed, uniform), Float64 1.05M on 256^3 255 / 244.  A forced layout keeps its
+// copy.
 bool gather_direct(const Mesh *m, int64_t n)
 {
     if (m->efi_layout) return false;
     const int64_t M = m->n[0] * m->n[1] * m->n[2];
-    const int64_t few = M / (m->dtype == SC_F32 ? 48 : 24);
-    return n <= (few > 100000 ? few : 100000);
+    const bool f32 = m->dtype == SC_F32;
+    int64_t few = f32 ? M / 11 : M / 6;
+    const int64_t most = f32 ? 190000 : 320000, least = f32 ? 125000 : 160000, far = M / (f32 ? 28 : 16);
+    few = few > most ? most : few < least ? least : few;
+    return n <= (few > far ? few : far);
 }
 
 int ensure_efi(Mesh *m)

@@ -23,9 +23,9 @@ def _uniform(n, T, k=3):
 
 
 @pytest.mark.parametrize("T,grid,few,many", [
-    (torch.float32, (32, 32, 32), 100_000, 100_001), (torch.float32, (128, 128, 128), 100_000, 340_000),
-    (torch.float32, (256, 256, 256), 349_525, 800_000), (torch.float64, (16, 16, 16), 1, 100_001),
-    (torch.float64, (100, 100, 100), 100_000, 250_000), (torch.float64, (128, 128, 128), 87_381, 690_000)])
+    (torch.float32, (32, 32, 32), 125_000, 125_001), (torch.float32, (128, 128, 128), 190_000, 340_000),
+    (torch.float32, (256, 256, 256), 599_186, 800_000), (torch.float64, (16, 16, 16), 1, 160_001),
+    (torch.float64, (100, 100, 100), 166_666, 250_000), (torch.float64, (128, 128, 128), 320_000, 690_000)])
 def test_field_copy_of_the_interpolation(T, grid, few, many):
     import spacecharge as sc
     mesh, copied = (sc.Mesh3D(grid, (-1.0,) * 3, (1.0,) * 3, T=T) for _ in range(2))
