@@ -48,13 +48,30 @@ constexpr int zconv_waves()
     return words > 32 || (CATH && (words > 20 || Shape<T, L>::E == 20)) ? 1 : CATH || words > 16 ? 2 : 3;
 }
 
-// The transposed convolution with the cathode image also holds the image sum;
-// for 20 Float64 values per lane on 320 points that spills (two registers of
-// 512), so the generic engine takes that one.
+// Whether the z convolution runs here: with the cathode image a lane holds the
+// image's spectrum (field) or sum (transposed) as well, three arrays of E values
+// beside the butterfly's temporaries, and at many values per lane the kernel drops to
+// one wave per SIMD and moves them through AGPRs; the generic kernel, which
+// splits a pencil over more lanes, is faster then and takes those lengths.
+// Measured (us, generic / this, 128x128 nodes across), field, Float64: 80 points
+// 96 / 135, 160 230 / 319, but 96 128 / 74, 200 309 / 161, 320 564 / 580 and even on
+// 90x90; in Float32 80 84 / 43, 160 143 / 155 and even on 90x90.  Transposed, Float64:
+// 80 119 / 173, 96 149 / 198, 160 265 / 393, 192 323 / 456, 200 339 / 408, 288 585 / 838,
+// 384 812 / 920 (320 spills two registers of 512), but 72 116 / 109, 144 247 / 249, 100
+// 160 / 164, 400 926 / 851; Float32: 80 92 / 146, 160 155 / 289, 200 211 / 219, 320 352 /
+// 623, 400 485 / 713, 256 (90x90) 141 / 155, but 96 101 / 39, 288 318 / 161.
 template <typename T, int L>
-constexpr bool adj_cathode_fits()
+constexpr bool zconv_here(int mode)
 {
-    return !(sizeof(T) == 8 && L == 320);
+    constexpr bool f64 = sizeof(T) == 8;
+    if (mode == kFieldCathode) return !(f64 && (L == 80 || L == 160));
+    if (mode != kAdjointCathode) return true;
+    switch (L) {
+    case 80: case 160: case 200: case 320: return false;
+    case 96: case 192: case 288: case 384: return !f64;
+    case 256: case 400: return f64;
+    default: return true;
+    }
 }
 
 // x pass of the real input: rows (y, z) of component blockIdx.y, zero-padded
@@ -463,8 +480,9 @@ void launch_all(Mesh *m, const Dims &d, int axis_kernel, const SolveIO &io)
         const cpx<T> *Gi = static_cast<const cpx<T> *>(ws.Gi);
         switch (io.mode) {
         case kFieldCathode:
-            hipLaunchKernelGGL((k_zconv_m<T, L, kFieldCathode>), zgrid, dim3(S::THREADS), 0, st, Fc, B, Gf,
-                               Gi, tw, d, (const SBunch *)nullptr, nbx);
+            if constexpr (zconv_here<T, L>(kFieldCathode))
+                hipLaunchKernelGGL((k_zconv_m<T, L, kFieldCathode>), zgrid, dim3(S::THREADS), 0, st, Fc, B,
+                                   Gf, Gi, tw, d, (const SBunch *)nullptr, nbx);
             break;
         case kPotential:
             hipLaunchKernelGGL((k_zconv_m<T, L, kPotential>), zgrid, dim3(S::THREADS), 0, st, Fc, B, Gf, Gi,
@@ -475,9 +493,9 @@ void launch_all(Mesh *m, const Dims &d, int axis_kernel, const SolveIO &io)
                                tw, d);
             break;
         case kAdjointCathode:
-            if constexpr (adj_cathode_fits<T, L>())
-            hipLaunchKernelGGL((k_zconv_adj_m<T, L, true>), zgrid, dim3(S::THREADS), 0, st, Fc, B, Gf, Gi,
-                               tw, d);
+            if constexpr (zconv_here<T, L>(kAdjointCathode))
+                hipLaunchKernelGGL((k_zconv_adj_m<T, L, true>), zgrid, dim3(S::THREADS), 0, st, Fc, B, Gf,
+                                   Gi, tw, d);
             break;
         default:
             hipLaunchKernelGGL((k_zconv_m<T, L, kFieldFree>), zgrid, dim3(S::THREADS), 0, st, Fc, B, Gf, Gi,
@@ -633,7 +651,7 @@ bool launch_mix(Mesh *m, int which, const SolveIO &io)
     switch (L) {
 #define X(LL) \
     case LL:                                                                   \
-        if (which == 2 && io.mode == kAdjointCathode && !adj_cathode_fits<T, LL>()) return false; \
+        if (which == 2 && !zconv_here<T, LL>(io.mode)) return false;               \
         launch_mix_length<T, LL>(m, d, which, io);                                 \
         return true;
         SC_MIX_LENGTHS(X)

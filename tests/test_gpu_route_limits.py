@@ -113,3 +113,36 @@ def test_padding_of_the_transforms(T, grid, halves):
         for c in range(3):
             d = (a[..., c] - b[..., c]).norm() / b[..., c].norm()
             assert float(d) <= (1e-5 if T == torch.float32 else 1e-12)
+
+
+# lengths along z at which the generic kernel is the faster one
+@pytest.mark.parametrize("kind,T,n", [
+    ("field", torch.float64, 40), ("field", torch.float64, 80), ("adjoint", torch.float64, 40),
+    ("adjoint", torch.float64, 96), ("adjoint", torch.float64, 192), ("adjoint", torch.float32, 40),
+    ("adjoint", torch.float32, 160), ("adjoint", torch.float32, 200)])
+def test_cathode_convolution_is_no_slower_than_the_generic_one(kind, T, n):
+    import spacecharge as sc
+    grid = (128, 128, n)
+    g = torch.rand((*grid, 3), device=DEV, dtype=T)
+    best, out = [], []
+    for generic in (False, True):
+        m = sc.Mesh3D(grid, (-1e-3, -1e-3, 1e-4), (1e-3, 1.2e-3, 2e-3), T=T, gamma=1.5)
+        m.force_generic_transforms(generic)
+        m.rho.copy_(g[..., 0])
+
+        def call():
+            if kind == "adjoint":
+                return sc.solve_adjoint(m, g, at_cathode=True)
+            sc.solve(m, at_cathode=True)
+            return m.efield
+        out.append(call().double())
+        times = []
+        for _ in range(5):
+            with sc.KernelTimer() as t:
+                for _ in range(4):
+                    call()
+            times.append(t.results()["zconv"][0])
+        best.append(min(times))
+    print(f"{kind} {T} {n}: {best[0]:.3f} ms, generic {best[1]:.3f}", flush=True)
+    assert float((out[0] - out[1]).norm() / out[1].norm()) <= (1e-5 if T == torch.float32 else 1e-12)
+    assert best[0] <= 1.15 * best[1]
