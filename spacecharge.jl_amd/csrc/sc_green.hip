@@ -1278,7 +1278,7 @@ bool green_fused(const Mesh *m, const Dims &d, size_t size, int cath)
 {
     if (smooth_lengths(m) || engine_of(m, d.Lx, false) == kGeneric) return false;
     const int64_t nodes = (int64_t)(d.nx + 1) * (d.ny + 1) * (cath ? d.nz + 1 + d.Lz : d.nz + 1);
-    return green_small(d, size, cath) || 24 * nodes > ((int64_t)256 << 20);
+    return green_small(m, d, size, cath) || 24 * nodes > ((int64_t)256 << 20);
 }
 
 template <typename T, int L>

@@ -391,7 +391,7 @@ int run_solve(Mesh *m, const double lo[3], const double hi[3], const double dl[3
     ws.deposited = false;
     bool overlap = false;
     if (!reuse) {
-        overlap = !ctx->in_batch && !green_small(d, sizeof(T), cath) &&
+        overlap = !ctx->in_batch && !green_small(m, d, sizeof(T), cath) &&
                   (cap ? ctx->side && ws.green_done && ws.deposit_start : ensure_side_stream(m) == SC_OK);
         if (overlap) {
             // the build forks where this step's deposit started (recorded by

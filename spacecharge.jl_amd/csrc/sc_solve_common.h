@@ -245,11 +245,22 @@ __device__ __forceinline__ void zconv_pencils(int task, int nbx, int Ly, int &bx
 // 10k particles on 16^3 on the side stream / inline 100 / 60 us, 100k on 32^3
 // 98 / 76, 200k on 48^3 Float32 115 / 104 but Float64 116 / 124, 1M on 64^3
 // 124 / 136; with the cathode 50k on 32^3 101 / 75, on 48^3 Float64 109 / 113.
-constexpr int64_t kSmallGreenBytes = 640 << 10;
-inline bool green_small(const Dims &d, size_t size, int cath)
+// Float64 particles on a Float32 mesh have generic passes on axes that are no powers
+// of two, and no fused kernel, and their builds take longer.  Two or three generic
+// passes: step of 2k such particles on 20^3 95 / 90, with the cathode 96 / 94, on 24^3
+// 96 / 97 and 97 / 102, 43x62x13 106 / 125, 33^3 107 / 122 (one solve 80 / 93), 21x244x23
+// 134 / 155 (96 / 125).  One: 32x32x20 and 64x64x20 level, of 60k on 32x32x50 104 / 112,
+// but one solve 70 / 60; on 50x64x32 99 / 116, one solve 68 / 70.
+constexpr int64_t kSmallGreenBytes = 640 << 10, kSmallWideBytes = 384 << 10, kSmallGenericBytes = 80 << 10;
+inline bool green_small(const Mesh *m, const Dims &d, size_t size, int cath)
 {
     const int64_t nodes = (int64_t)(d.nx + 1) * (d.ny + 1) * (d.nz + 1);
-    return nodes * (int64_t)size * (cath ? 2 : 1) <= kSmallGreenBytes;
+    int generic = 0;
+    for (const int L : {d.Lx, d.Ly, d.Lz}) generic += engine_of(m, L, false) == kGeneric;
+    const int64_t most = generic > 1                            ? kSmallGenericBytes
+                         : generic > 0 && smooth_lengths(m) ? kSmallWideBytes
+                                                                : kSmallGreenBytes;
+    return nodes * (int64_t)size * (cath ? 2 : 1) <= most;
 }
 
 // Builds the transformed Green functions for green_mode `mode` into ws.Gf

@@ -3,6 +3,8 @@ launch counts of the library's kernel timers.  Particles that fill the mesh meas
 slower on the path for few particles from a little beyond the limits on."""
 from __future__ import annotations
 
+import ctypes
+
 import pytest
 import torch
 
@@ -113,6 +115,42 @@ def test_padding_of_the_transforms(T, grid, halves):
         for c in range(3):
             d = (a[..., c] - b[..., c]).norm() / b[..., c].norm()
             assert float(d) <= (1e-5 if T == torch.float32 else 1e-12)
+
+
+def _forks(call):
+    """Whether the captured call runs kernels beside each other."""
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        call()
+    hip = ctypes.CDLL("libamdhip64.so")
+    nodes, edges = ctypes.c_size_t(), ctypes.c_size_t()
+    g = ctypes.c_void_p(graph.raw_cuda_graph())
+    assert hip.hipGraphGetNodes(g, None, ctypes.byref(nodes)) == 0
+    assert hip.hipGraphGetEdges(g, None, None, ctypes.byref(edges)) == 0
+    return edges.value >= nodes.value  # a chain has one edge fewer than nodes
+
+
+# a Green build with generic passes beside the deposit, on the caller's stream only
+# where it is smaller than one of the register engines
+@pytest.mark.parametrize("T,P,grid,beside", [
+    (torch.float32, torch.float64, (20, 20, 20), False), (torch.float32, torch.float64, (33, 33, 33), True),
+    (torch.float32, torch.float64, (100, 20, 20), True), (torch.float32, torch.float64, (32, 32, 32), False),
+    (torch.float32, torch.float64, (50, 64, 32), True), (torch.float32, torch.float64, (32, 32, 50), False),
+    (torch.float32, torch.float64, (64, 64, 64), True), (torch.float32, torch.float32, (33, 33, 33), False),
+    (torch.float64, torch.float64, (300, 8, 8), False), (torch.float64, torch.float64, (48, 48, 48), True)])
+def test_stream_of_the_green_build(T, P, grid, beside):
+    import spacecharge as sc
+    mesh, big = (sc.Mesh3D(g, (-1.0,) * 3, (1.0,) * 3, T=T) for g in (grid, (64, 64, 64)))
+    p = _uniform(3000, P, 4)
+    for m in (big, mesh):  # the larger one makes the library's second stream
+
+        def step(m=m):
+            p[3].mul_(1.0)  # one first node of the graph
+            sc.deposit(m, *p)
+            sc.solve(m)
+        step()
+    torch.cuda.synchronize()
+    assert _forks(step) == beside
 
 
 # lengths along z at which the generic kernel is the faster one
