@@ -42,27 +42,27 @@ inline Split split_of(int64_t n, int slice_log2, int ntiles)
 
 // Most particles that the direct deposit takes on a mesh of T tiles (0: none),
 // f32 the mesh type, nchan charge channels.  Its cost grows with the particle-tile
-// pairs and with the sub-grids, the binned chain's hardly; particles that fill
-// the mesh are the binned chain's best case, so the line lies below where those
-// break even.  Measured (replayed from a graph, uniform particles, direct / binned,
-// us), Float64: 10k on 16^3 7.7 / 37; 8 tiles, 262k (2M pairs) 27.6 / 48.7, 524k 37 /
-// 51, 734k 67 / 52; 27 tiles, 155k (4M pairs) 41.5 / 42.9, 217k 49.5 / 48; 64 tiles,
-// 33k (2M pairs) 29.6 / 35.7, 46k 36.1 / 36.2, 66k 49.7 / 36.9.  Float32, with one
-// launch more and a cheaper chain: 10k on 16^3 13 / 32; 8 tiles, 262k 31 / 41, 524k
-// 40 / 45, 734k 60 / 46; 27 tiles, 54k (1.4M pairs) 27.6 / 32, 78k (2M) 38 / 33; 64
-// tiles, 23k (1.4M) 31.5 / 32.6, 46k 40 / 33.  One tile has no pairs to spare: there
-// only the size of the sub-grids ends the range.  Three channels triple the
-// sub-grids and share one binning: 4k on 64 tiles 50 / 39 in Float32, 44.7 / 43.2 in
-// Float64, 9k on 27 tiles 35.8 / 33.9 in Float32; Float64 on 4 tiles, 245k (2.8M) 35 /
-// 53, 350k 57 / 52.
+// pairs and with the sub-grids, the binned chain's hardly; but it is two or three
+// launches, the chain six, and a step of so few particles waits for the host as
+// often as for the GPU.  Deposit alone (replayed from a graph, uniform particles, the
+// chain's best case, direct / binned, us), Float64: 10k on 16^3 7.7 / 37; 8 tiles, 524k 37 /
+// 51, 734k 67 / 52; 27 tiles, 217k (5.6M pairs) 49.5 / 48; 64 tiles, 66k (4M) 49.7 / 36.9.
+// Float32: 10k on 16^3 13 / 32; 8 tiles, 524k 40 / 45; 27 tiles, 78k (2M) 38 / 33; 64
+// tiles, 23k 31.5 / 32.6, 46k 40 / 33.  Steps (uniform, then rms a tenth of the mesh),
+// Float64: 64 tiles, 42k 103 / 105 and 101 / 107, 55k (3.4M) 105 / 105 and 102 / 109, 65k
+// 111 / 106 and 108 / 110; 48 tiles, 60k 99 / 104 and 97 / 106, 87k (4M) 111 / 104 and 102 /
+// 106; 36 tiles, 75k 89 / 95 and 88 / 98.  Float32: 18 tiles, 116k (2M) 76 / 84 and 75 /
+// 87; 27 tiles, 77k 87 / 89 and 89 / 97; 64 tiles, 32k 87 / 96 and 87 / 98.  Three
+// channels triple the sub-grids and share one binning, so that replayed from a graph
+// they lose sooner (Float32, 27 tiles, 13k 44 / 41 and 41 / 48; 64 tiles, 8k 59 / 48 and
+// 53 / 46; Float64, 64 tiles, 16k 60 / 57), but the gradient step that they are part
+// of gains (Float32, 27 tiles, 26k 179 / 181 and 187 / 194; 64 tiles, 11k 190 / 209; Float64, 64
+// tiles, 16k 218 / 229, 22k 234 / 228; 36 tiles, 39k 186 / 206).  One tile has no pairs to
+// spare: there only the size of the sub-grids ends the range.
 inline int64_t direct_most(int T, bool f32, int nchan)
 {
     constexpr int64_t k = (int64_t)1 << 20;
-    const int64_t pairs = T == 1 ? 16 * k : f32 ? (T <= 8 ? 2 * k : 7 * k / 5) : T <= 32 ? 4 * k : 5 * k / 2;
-    if (nchan > 1 && T > 1) {
-        if (T > (f32 ? 8 : 32)) return 0;
-        if (pairs > 3 * k) return 3 * k / ((int64_t)T * nchan);
-    }
+    const int64_t pairs = T == 1 ? 16 * k : f32 ? 2 * k : T <= 32 ? 4 * k : 7 * k / 2;
     return T > kDirectTiles ? 0 : pairs / ((int64_t)T * nchan);
 }
 

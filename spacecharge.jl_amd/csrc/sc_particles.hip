@@ -105,7 +105,11 @@ struct V4<double> {
 // last-level cache as it grows.  Measured (copy and gather, us), Float64, P = 1 /
 // node pairs padded to 64 bytes, an earlier layout / P = 2: 4M particles on 128^3
 // - / 231 / 173, the 2M cathode bunch on 64x64x128 - / 99 / 73, 1M on 64^3 53 / 49
-// / 38, 8M on 256^3 944 / 1243 / 750: packed for every Float64 mesh.  Float32, where
+// / 38, 8M on 256^3 944 / 1243 / 750: packed for every Float64 mesh.  (Bunches with a
+// core, in one way or another; particles that fill the mesh evenly go from 4% faster
+// than node pairs (2M on 160^3 240 / 228) to 10% slower (4M on 128^3 350 / 384, 1.5M on
+// 100^3 126 / 131), where those with a core, rms a tenth of the mesh, go 24-31% faster.)
+// Float32, where
 // a run of six straddles its 16-byte loads, P = 1 / 2: 2M on 64^3 48 / 44, 8M on
 // 64x64x128 174 / 155, but 4M on 128^3 104 / 108, 8M on 128x128x256 235 / 240 and
 // even between; then 2M on 160^3 78 / 75, 4M on 200^3 183 / 162, 8M on 256^3 514 /

@@ -1,6 +1,5 @@
 """GPU: which path a call takes around the limits of the dispatch rules, from the
-launch counts of the library's kernel timers.  Particles that fill the mesh measured
-slower on the path for few particles from a little beyond the limits on."""
+launch counts of the library's kernel timers."""
 from __future__ import annotations
 
 import ctypes
@@ -43,9 +42,9 @@ def test_field_copy_of_the_interpolation(T, grid, few, many):
 
 @pytest.mark.parametrize("T,grid,few,many", [
     (torch.float32, (16, 16, 16), 1_000_000, 17_000_000), (torch.float32, (32, 32, 32), 262_144, 734_000),
-    (torch.float32, (48, 48, 48), 54_370, 77_672), (torch.float32, (64, 64, 64), 22_937, 32_768),
+    (torch.float32, (48, 48, 48), 77_672, 77_673), (torch.float32, (64, 64, 64), 32_768, 32_769),
     (torch.float64, (32, 32, 32), 524_288, 734_000), (torch.float64, (48, 48, 48), 155_344, 217_482),
-    (torch.float64, (64, 64, 64), 40_960, 65_536), (torch.float64, (65, 65, 81), 20_000, 40_000)])
+    (torch.float64, (64, 64, 64), 57_344, 65_536), (torch.float64, (65, 65, 81), 20_000, 40_000)])
 def test_binning_of_the_deposit(T, grid, few, many):
     import spacecharge as sc
     mesh, binned = (sc.Mesh3D(grid, (-1.0,) * 3, (1.0,) * 3, T=T) for _ in range(2))
@@ -63,15 +62,13 @@ def test_binning_of_the_deposit(T, grid, few, many):
 
 
 @pytest.mark.parametrize("T,grid,few,many", [
-    (torch.float32, (32, 32, 32), 87_381, 174_762), (torch.float32, (48, 48, 48), 0, 9061),
-    (torch.float64, (33, 33, 17), 244_667, 349_525), (torch.float64, (64, 64, 64), 0, 3822)])
+    (torch.float32, (32, 32, 32), 87_381, 174_762), (torch.float32, (48, 48, 48), 25_890, 25_891),
+    (torch.float64, (33, 33, 17), 349_525, 349_526), (torch.float64, (64, 64, 64), 19_114, 21_846)])
 def test_binning_of_the_cotangent_deposit(T, grid, few, many):
     import spacecharge as sc
     mesh, binned = (sc.Mesh3D(grid, (-1.0,) * 3, (1.0,) * 3, T=T) for _ in range(2))
     binned.set_deposit_tiling(13, 11)
     for n in (few, many):
-        if not n:
-            continue
         p = _uniform(n, T, 6)
         got = []
         assert _launched(lambda: got.append(sc.interpolate_adjoint(mesh, *p, positions=False)[0]),
