@@ -1082,8 +1082,9 @@ k_green_3m(const T *__restrict__ R, T *__restrict__ Gf, cpx<T> *__restrict__ Gi,
 // the x transform in place.  The node rows that neighbouring workgroups share
 // are evaluated twice (1/S more, and 1/K more along z for K planes).
 // The terms and their order are k_green_f3's; the column and row logs of a plane
-// come from LDS tables, as does log(u^2 + v^2) of each node (one node at a time per lane: with a lane's nodes unrolled the kernel
-// took 238 VGPRs instead of 192 at 256 points and the 128^3 build 79 us, not 75).
+// come from LDS tables, as does log(u^2 + v^2) of each node (one node at a time
+// per lane: with a lane's nodes unrolled the kernel took 238 VGPRs instead of 192
+// at 256 points and the 128^3 build 79 us, not 75).
 // Squares and their sums are rounded one by one: with the compiler's choice of
 // fused forms, which differed between r and the tables, the field of a Float64
 // mesh lay 4-5% further from a plain 64-bit evaluation than with k_green_f3
